@@ -220,131 +220,228 @@ __global__ __launch_bounds__(kBlock) void k_ffnn(const float* __restrict__ Wg, c
     }
 }
 
-// FP32 network for few pairs: one 16-pair tile per block, and the block's waves take the 16-unit
-// blocks of every layer between them (wave w computes blocks MPW w .. MPW w + MPW - 1 of every
-// hidden layer and of every backward delta, over all k-steps), so that a tile's chain of layers is
-// spread over MT / MPW waves instead of running on one.  The layer outputs go through LDS to the
-// next layer's B operands.  Every accumulator takes the same products in the same order as
-// ffnn_tiles, and the output sum is formed the same way, so E and dE/dG equal k_ffnn's bit for
-// bit.  One block per wave (MPW = 1): the 640-thread block of a 160-wide network needs 131 VGPRs
-// per lane, within the 168 that three waves per SIMD leave; each layer's weight reads are kept in
-// that layer, or the compiler hoists them all and spills.
-template <class N>
-constexpr int coop_mpw() { return 1; }
-
+// FP32 network with the layers' unit blocks spread over a block's waves.  Wave w computes 16-unit
+// block w of every hidden layer and of every backward delta for the block's NT tiles of 16 pairs, over
+// all k-steps; the layer outputs go through LDS to the next layer's B operands.  The bound is the FP32
+// matrix rate once a weight operand read from L2 (256 bytes for the wave) serves several products:
+// one wave per tile read the whole network (780 KB for 121 -> 150 x 4) for every 16 pairs.  NT tiles
+// share each operand read, and the operands are loaded kDepth chunks ahead, across the layers'
+// barriers, so that L2 latency is covered even with one tile per block.  Every accumulator takes the
+// same products in the same order as ffnn_tiles, and the output sum is formed the same way, so E and
+// dE/dG equal k_ffnn's bit for bit, for any NT.  121 -> 150 x 4: 241 rows 46 -> 18 us, 100,001 rows
+// 1,960 -> 406 us (96 TFLOP/s of padded products, 0.65 of the FP32 rate a large matrix product reaches).
 template <class N, int ACT>
-__global__ __launch_bounds__(N::MT / coop_mpw<N>() * 64) void k_ffnn_coop(
-    const float* __restrict__ W, float en_min, float scale, int D, const float* __restrict__ G,
-    const int32_t* __restrict__ np_dev, int64_t maxp, float* __restrict__ E, float* __restrict__ dEdG) {
+struct SpreadNet {
+    static constexpr int MT = N::MT, NL = N::NL, BLOCK = 64 * MT;
+    // ReLU keeps one bit per hidden unit for the backward pass, tanh the activation itself
+    static constexpr int NT = (ACT == NEPX_ACT_RELU || NL <= 2) ? 4 : 2;
+    static constexpr int BLOCKS_PER_CU = 2;  // LDS and registers allow two; each hides the other's barriers
+    static constexpr int WAVES_PER_SIMD = (BLOCKS_PER_CU * MT + 3) / 4;
+    // products in order: forward layers 0..NL-1, backward layers NL-1..0; chunks of four k-steps
+    static constexpr int chunks(int q) { return (q == 0 ? N::KD : N::KH) / 4; }
+    static constexpr int first(int q) { return q == 0 ? 0 : first(q - 1) + chunks(q - 1); }
+    static constexpr int TOTAL = first(2 * NL);
+    static constexpr int product_of(int f) {
+        int q = 0;
+        while (f >= first(q + 1)) ++q;
+        return q;
+    }
+};
+// Operand chunks in flight per wave: the fewer products a chunk feeds, the further ahead it is read.
+constexpr int spread_depth(int nt) { return nt >= 4 ? 3 : nt == 2 ? 4 : 6; }
+
+template <int COUNT, int I = 0, class Fn>
+__device__ __forceinline__ void static_for(Fn&& fn) {
+    if constexpr (I < COUNT) {
+        fn(std::integral_constant<int, I>{});
+        static_for<COUNT, I + 1>(fn);
+    }
+}
+
+template <class N, int ACT, int NT>
+__device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float en_min, float scale, int D,
+                                            const float* __restrict__ G, int P, int tile0, float* __restrict__ E,
+                                            float* __restrict__ dEdG,
+                                            v4f (&xs)[2][SpreadNet<N, ACT>::NT][N::MT][64]) {
+    using S = SpreadNet<N, ACT>;
     constexpr NetLayout Lay = N::layout();
-    constexpr int MT = N::MT, MPW = coop_mpw<N>();
-    static_assert(MT % MPW == 0, "unit blocks split evenly over the waves");
-    __shared__ v4f xs[2][MT][64];  // one layer's outputs: block c of lane l at [c][l]
-    const int P = n_pairs(np_dev, maxp);
-    int lane = threadIdx.x & 63;
-    asm volatile("" : "+v"(lane));  // keeps the weight reads inside the tile loop
-    const int g = lane >> 4;
-    const int m0 = (threadIdx.x >> 6) * MPW;  // this wave's first 16-unit block
-    const int nt = (P + 15) / 16;
-    for (int tile = blockIdx.x; tile < nt; tile += gridDim.x) {
-        const int p = tile * 16 + (lane & 15);
-        v4f gin[N::MD];
-        gather_chunks<N::MD>(G + (size_t)p * D, p < P, D, gin);
-        v4f hown[N::NL][MPW];  // this wave's blocks of every hidden layer
-        int buf = 0;
+    constexpr int MT = N::MT, NL = N::NL, kDepth = spread_depth(NT);
+    uint32_t lane = threadIdx.x;
+    asm volatile("" : "+v"(lane));  // keeps the operand reads inside the caller's loop
+    lane &= 63u;                    // known range: the reads take a scalar base and this offset
+    const int g = lane >> 4, pl = lane & 15;
+    const int m = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // this wave's 16-unit block
+    // operands of chunk f of the whole sequence for this wave's block (dE/dG has MD blocks only: the
+    // other waves read block 0's there and drop out before using them)
+    float ring[kDepth][4];
+    auto load_chunk = [&](auto fc) {
+        constexpr int f = decltype(fc)::value;
+        if constexpr (f < S::TOTAL) {
+            constexpr int q = S::product_of(f), c = f - S::first(q);
+            constexpr int k = q < NL ? q : 2 * NL - 1 - q;
+            constexpr int ks = q == 0 ? N::KD : N::KH;
+            constexpr int off = (q < NL ? Lay.fwd_off(k) : Lay.bwd_off(k)) + 4 * c * 64;
+            const int mm = (q == 2 * NL - 1 && N::MD < MT && m >= N::MD) ? 0 : m;
+            const float* src = W + (off + mm * ks * 64);
 #pragma unroll
-        for (int k = 0; k < N::NL; ++k) {
-            asm volatile("" : "+v"(lane));  // each layer's weight reads stay in that layer
-            const float* Wf = W + Lay.fwd_off(k);
-            const int ks = (k == 0) ? N::KD : N::KH;
-            v4f acc[MPW];
-#pragma unroll
-            for (int i = 0; i < MPW; ++i) {
-                const float4 b4 = *reinterpret_cast<const float4*>(W + Lay.bias_off(k) + 16 * (m0 + i) + 4 * g);
-                acc[i] = v4f{b4.x, b4.y, b4.z, b4.w};
-            }
-#pragma unroll
-            for (int c = 0; c < ks / 4; ++c) {
-                const v4f x = (k == 0) ? gin[c < N::MD ? c : 0] : xs[buf ^ 1][c][lane];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int i = 0; i < MPW; ++i)
-                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(Wf[((m0 + i) * ks + 4 * c + r) * 64 + lane],
-                                                                     x[r], acc[i], 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < MPW; ++i) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) hown[k][i][r] = act_fwd(acc[i][r], ACT);
-                xs[buf][m0 + i][lane] = hown[k][i];
-            }
-            __syncthreads();
-            buf ^= 1;
+            for (int r = 0; r < 4; ++r) ring[f % kDepth][r] = src[r * 64 + lane];
         }
-        // output layer: every wave forms y from the whole last layer, in ffnn_tiles' order
+    };
+    auto load4 = [&](const float* src) {  // units 16 m + 4 g + 0..3 of a bias or the output layer
+        const float4 v = *reinterpret_cast<const float4*>(src + 16 * m + 4 * g);
+        return v4f{v.x, v.y, v.z, v.w};
+    };
+    v4f bias = load4(W + Lay.bias_off(0));  // one layer ahead
+    static_for<kDepth>([&](auto f) { load_chunk(f); });
+    // the input rows in the B operand's layout: wave c loads chunk c
+    if (m < N::MD) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int p = (tile0 + t) * 16 + pl;
+            v4f v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = 16 * m + 4 * g + r;
+                v[r] = (p < P && e < D) ? G[(size_t)p * D + e] : 0.f;
+            }
+            xs[0][t][m][lane] = v;
+        }
+    }
+    __syncthreads();
+    // acc += the product q of this wave's block with the vectors in xs[buf]
+    auto product = [&](auto qc, v4f (&acc)[NT]) {
+        constexpr int q = decltype(qc)::value, buf = (q < NL ? q : q + 1) & 1;
+        v4f x[2][NT];  // one chunk ahead
+#pragma unroll
+        for (int t = 0; t < NT; ++t) x[0][t] = xs[buf][t][0][lane];
+        static_for<S::chunks(q)>([&](auto cc) {
+            constexpr int c = decltype(cc)::value, f = S::first(q) + c;
+            if constexpr (c + 1 < S::chunks(q)) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) x[(c + 1) & 1][t] = xs[buf][t][c + 1][lane];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ring[f % kDepth][r], x[c & 1][t][r], acc[t], 0, 0, 0);
+            load_chunk(std::integral_constant<int, f + kDepth>{});
+            __builtin_amdgcn_sched_barrier(0);  // reads stay this far ahead; all at once they would spill
+        });
+    };
+    constexpr bool BITS = ACT == NEPX_ACT_RELU;
+    v4f h[BITS ? 1 : NL][BITS ? 1 : NT];  // this wave's activations (tanh)
+    uint32_t on[BITS ? NL : 1] = {};      // its active units (ReLU), bit 4 t + r
+    auto der = [&](int k, int t, int r) {
+        if constexpr (BITS) return (on[k] >> (4 * t + r)) & 1u ? 1.f : 0.f;
+        else return act_der(h[k][t][r], ACT);
+    };
+    static_for<NL>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        v4f acc[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = bias;
+        bias = load4(W + (k + 1 < NL ? Lay.bias_off(k + 1) : Lay.wout_off()));
+        product(kc, acc);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            v4f o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                o[r] = act_fwd(acc[t][r], ACT);
+                if constexpr (BITS) on[k] |= (o[r] > 0.f ? 1u : 0u) << (4 * t + r);
+            }
+            if constexpr (!BITS) h[k][t] = o;
+            xs[(k + 1) & 1][t][m][lane] = o;
+        }
+        __syncthreads();
+    });
+    // the last layer's deltas (`bias` holds the output layer's weights of this wave's units)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        v4f d;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[r] = scale * bias[r] * der(NL - 1, t, r);
+        xs[(NL + 1) & 1][t][m][lane] = d;
+    }
+    // output layer: wave t forms tile t's sum from the whole last layer, in ffnn_tiles' order
+    if (m < NT) {
         const float* wo = W + Lay.wout_off();
         float y = 0.f;
 #pragma unroll
         for (int c = 0; c < MT; ++c) {
             const float4 w4 = *reinterpret_cast<const float4*>(wo + 16 * c + 4 * g);
             const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
-            const v4f h = xs[buf ^ 1][c][lane];
+            const v4f hv = xs[NL & 1][m][c][lane];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) y += wv[r] * h[r];
+            for (int r = 0; r < 4; ++r) y += wv[r] * hv[r];
         }
         y += __shfl_xor(y, 16);
         y += __shfl_xor(y, 32);
         y += W[Lay.bout_off()];
-        if (m0 == 0 && p < P && lane < 16) E[p] = en_min + scale * y;
-        v4f delta[MPW];
+        const int p = (tile0 + m) * 16 + pl;
+        if (p < P && lane < 16) E[p] = en_min + scale * y;
+    }
+    __syncthreads();
+    static_for<NL - 1>([&](auto jc) {  // the deltas of layer k - 1 from those of layer k
+        constexpr int q = NL + decltype(jc)::value, k = 2 * NL - 1 - q;
+        v4f acc[NT];
 #pragma unroll
-        for (int i = 0; i < MPW; ++i) {
-            const float4 w4 = *reinterpret_cast<const float4*>(wo + 16 * (m0 + i) + 4 * g);
-            const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
+        for (int t = 0; t < NT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+        product(std::integral_constant<int, q>{}, acc);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) delta[i][r] = scale * wv[r] * act_der(hown[N::NL - 1][i][r], ACT);
+        for (int t = 0; t < NT; ++t) {
+            v4f d;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) d[r] = acc[t][r] * der(k - 1, t, r);
+            xs[q & 1][t][m][lane] = d;
         }
-        // backward: layer k's deltas through LDS, then this wave's blocks of layer k-1 (k = 0: dE/dG)
+        __syncthreads();
+    });
+    if (m < N::MD) {  // dE/dG (uniform per wave)
+        v4f acc[NT];
 #pragma unroll
-        for (int k = N::NL - 1; k >= 0; --k) {
+        for (int t = 0; t < NT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+        product(std::integral_constant<int, 2 * NL - 1>{}, acc);
 #pragma unroll
-            for (int i = 0; i < MPW; ++i) xs[buf][m0 + i][lane] = delta[i];
-            __syncthreads();
-            buf ^= 1;
-            if (k == 0 && m0 >= N::MD) break;
-            asm volatile("" : "+v"(lane));
-            const float* Wb = W + Lay.bwd_off(k);
-            const int mtn = (k == 0) ? N::MD : MT;  // output blocks of this product
-            v4f acc[MPW];
+        for (int t = 0; t < NT; ++t) {
+            const int p = (tile0 + t) * 16 + pl;
 #pragma unroll
-            for (int i = 0; i < MPW; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < N::KH / 4; ++c) {
-                const v4f x = xs[buf ^ 1][c][lane];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int i = 0; i < MPW; ++i)
-                        if (m0 + i < mtn)
-                            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                Wb[((m0 + i) * N::KH + 4 * c + r) * 64 + lane], x[r], acc[i], 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < MPW; ++i) {
-                if (k > 0) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) delta[i][r] = acc[i][r] * act_der(hown[k - 1][i][r], ACT);
-                } else if (m0 + i < N::MD) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int e = 16 * (m0 + i) + 4 * g + r;
-                        if (p < P && e < D) dEdG[(size_t)p * D + e] = acc[i][r];
-                    }
-                }
+            for (int r = 0; r < 4; ++r) {
+                const int e = 16 * m + 4 * g + r;
+                if (p < P && e < D) dEdG[(size_t)p * D + e] = acc[t][r];
             }
         }
-        __syncthreads();  // the last reads of xs are done before the next tile writes it
+    }
+}
+
+// Each block takes an equal run of tiles, in groups of NT, then of two and one: with many pairs the
+// operand reads are shared four ways and the blocks end together, with few every block has one tile.
+template <class N, int ACT>
+__global__ __launch_bounds__((SpreadNet<N, ACT>::BLOCK)) __attribute__((
+    amdgpu_waves_per_eu(SpreadNet<N, ACT>::WAVES_PER_SIMD, SpreadNet<N, ACT>::WAVES_PER_SIMD))) void k_ffnn_spread(
+    const float* __restrict__ W, float en_min, float scale, int D, const float* __restrict__ G,
+    const int32_t* __restrict__ np_dev, int64_t maxp, float* __restrict__ E, float* __restrict__ dEdG) {
+    using S = SpreadNet<N, ACT>;
+    __shared__ v4f xs[2][S::NT][N::MT][64];  // one layer's outputs: block c of lane l of tile t at [t][c][l]
+    const int P = n_pairs(np_dev, maxp);
+    const int nt = (P + 15) / 16;
+    const int per = (nt + gridDim.x - 1) / gridDim.x;
+    int tile = blockIdx.x * per;
+    const int end = tile + per < nt ? tile + per : nt;
+    while (tile < end) {  // uniform over the block
+        const int left = end - tile;
+        if (S::NT >= 4 && left >= 4) {
+            ffnn_spread<N, ACT, S::NT>(W, en_min, scale, D, G, P, tile, E, dEdG, xs);
+            tile += 4;
+        } else if (left >= 2) {
+            ffnn_spread<N, ACT, 2>(W, en_min, scale, D, G, P, tile, E, dEdG, xs);
+            tile += 2;
+        } else {
+            ffnn_spread<N, ACT, 1>(W, en_min, scale, D, G, P, tile, E, dEdG, xs);
+            tile += 1;
+        }
+        __syncthreads();  // the last reads of xs are done before the next tiles write it
     }
 }
 
@@ -800,42 +897,43 @@ static void launch_ffnn_p(const nepx_net* net, int grid, float scale, int d, con
 template <class T, int NT>
 static int launch_ffnn(const nepx_net* net, int grid, float scale, int d, const float* G, const int32_t* np_dev,
                        int64_t maxp, float* E, float* dEdG, void* stream) {
-    if constexpr (T::HP % 32 == 0) {
-        switch (net->precision) {
-            case NEPX_NET_F16X3:
-                launch_ffnn_p<T, NT, NEPX_NET_F16X3>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
-                break;
-            case NEPX_NET_BF16:
-                launch_ffnn_p<T, NT, NEPX_NET_BF16>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
-                break;
-            case NEPX_NET_BF16X3:
-                launch_ffnn_p<T, NT, NEPX_NET_BF16X3>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
-                break;
-            default:
+    switch (net->precision) {
+        case NEPX_NET_F16X3:
+            launch_ffnn_p<T, NT, NEPX_NET_F16X3>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
+            break;
+        case NEPX_NET_BF16:
+            launch_ffnn_p<T, NT, NEPX_NET_BF16>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
+            break;
+        case NEPX_NET_BF16X3:
+            launch_ffnn_p<T, NT, NEPX_NET_BF16X3>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
+            break;
+        default:  // networks too wide for LDS run on k_ffnn_spread
+            if constexpr (weights_in_lds<T, NEPX_NET_F32>())
                 launch_ffnn_p<T, NT, NEPX_NET_F32>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
-        }
-    } else {
-        launch_ffnn_p<T, NT, NEPX_NET_F32>(net, grid, scale, d, G, np_dev, maxp, E, dEdG, stream);
     }
     NEPX_LAUNCH_CHECK();
     return NEPX_OK;
 }
 
-// Few tiles (up to four per CU): the FP32 network runs one tile per block on k_ffnn_coop, which gives
-// the same results as k_ffnn.
+// The FP32 network runs on k_ffnn_spread where a block's copy of its operands does not fit in LDS (one
+// wave per tile would read them from L2 for every tile: 60 -> 128 x 2 at 20,000 rows 93 us against
+// 28, 121 -> 150 x 4 536 against 97), and, for the network that fits, up to four tiles per CU (too few
+// for a wave each; beyond, k_ffnn's copy in LDS is as fast); same results.
 template <class T>
-static bool launch_ffnn_coop(const nepx_net* net, float scale, int d, const float* G, const int32_t* np_dev,
-                             int64_t maxp, float* E, float* dEdG, void* stream) {
-    const bool f32 = net->precision == NEPX_NET_F32 || T::HP % 32 != 0;
-    const int64_t tiles = (maxp + 15) / 16;
-    if (!f32 || tiles > 4 * (int64_t)device_cus()) return false;
-    const dim3 grid((unsigned)tiles), block(T::MT / coop_mpw<T>() * 64);
-    if (net->act == NEPX_ACT_TANH)
-        hipLaunchKernelGGL((k_ffnn_coop<T, NEPX_ACT_TANH>), grid, block, 0, as_stream(stream), net->w_packed,
-                           net->en_min, scale, d, G, np_dev, maxp, E, dEdG);
-    else
-        hipLaunchKernelGGL((k_ffnn_coop<T, NEPX_ACT_RELU>), grid, block, 0, as_stream(stream), net->w_packed,
-                           net->en_min, scale, d, G, np_dev, maxp, E, dEdG);
+static bool launch_ffnn_spread(const nepx_net* net, float scale, int d, const float* G, const int32_t* np_dev,
+                               int64_t maxp, float* E, float* dEdG, void* stream) {
+    const int64_t tiles = (maxp + 15) / 16, cus = device_cus();
+    if (net->precision != NEPX_NET_F32 || (weights_in_lds<T, NEPX_NET_F32>() && tiles > 4 * cus)) return false;
+#define NEPX_LAUNCH_SPREAD(A)                                                                                   \
+    hipLaunchKernelGGL((k_ffnn_spread<T, A>),                                                                   \
+                       dim3((unsigned)(tiles < SpreadNet<T, A>::BLOCKS_PER_CU * cus                             \
+                                           ? tiles                                                              \
+                                           : SpreadNet<T, A>::BLOCKS_PER_CU * cus)),                            \
+                       dim3(SpreadNet<T, A>::BLOCK), 0, as_stream(stream), net->w_packed, net->en_min, scale, d, G, \
+                       np_dev, maxp, E, dEdG)
+    if (net->act == NEPX_ACT_TANH) NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH);
+    else NEPX_LAUNCH_SPREAD(NEPX_ACT_RELU);
+#undef NEPX_LAUNCH_SPREAD
     return true;
 }
 
@@ -851,7 +949,7 @@ extern "C" int nepx_ffnn_fwd_bwd(const nepx_net* net, const float* G, const int3
     const float scale = net->en_max - net->en_min;
 #define X(d, w, h, T, NT)                                                                        \
     if (net->d_in == d && net->width == w && net->n_hidden == h) {                               \
-        if (launch_ffnn_coop<T>(net, scale, d, G, np_dev, maxp, E, dEdG, stream)) {              \
+        if (launch_ffnn_spread<T>(net, scale, d, G, np_dev, maxp, E, dEdG, stream)) {              \
             NEPX_LAUNCH_CHECK();                                                                 \
             return NEPX_OK;                                                                      \
         }                                                                                        \

@@ -127,6 +127,28 @@ def test_ffnn_few_pairs_kernel_equals_wide_kernel(gpu, d_in, widths, act):
     assert normwise_rel(E0, -2.0 + 5.0 * y) < 1e-5 and normwise_rel(g0, 5.0 * g) < 1e-4
 
 
+@pytest.mark.parametrize("d_in,widths,act", [(121, [150] * 4, "relu"), (121, [150] * 4, "tanh"),
+                                             (47, [150] * 4, "relu"), (60, [128, 128], "tanh")])
+def test_ffnn_tile_groups_equal_single_tiles(gpu, d_in, widths, act):
+    """The FP32 network's blocks take equal runs of 16-pair tiles in groups of four, two and one (512
+    blocks on 256 CUs: 3, 5 and 7 tiles per block here, the last row short of a tile); every row equals,
+    bit for bit, the same row of a call small enough for one tile per block."""
+    import nepx
+    from nepx import ops
+    net = nepx.EnergyNet.random(d_in, widths, seed=5, act=act, en_min=-2.0, en_max=3.0, device=gpu, precision="f32")
+    g = torch.Generator(device=gpu).manual_seed(4)
+    for per_block in (3, 5, 7):
+        P = 16 * 512 * per_block - 5
+        G = 20.0 * torch.rand((P, d_in), generator=g, device=gpu)
+        E, dG = ops.ffnn_forward_backward(net, G)
+        for a in (0, P // 2, P - 4001):
+            e, d = ops.ffnn_forward_backward(net, G[a:a + 4001].contiguous())
+            assert torch.equal(E[a:a + 4001], e) and torch.equal(dG[a:a + 4001], d)
+        y, want = O.ffnn_forward_backward(G[-500:].cpu().numpy().astype(np.float64), net.layers_f64(), act)
+        assert normwise_rel(E[-500:].cpu().numpy(), -2.0 + 5.0 * y) < 1e-5
+        assert normwise_rel(dG[-500:].cpu().numpy(), 5.0 * want) < 1e-4
+
+
 def test_ffnn_split_large_inputs_and_energy_range(gpu):
     """The fp16 hi/lo path with descriptor entries up to 4000 (|G| <= Nd^2 bounds real rows far
     below fp16's 65504) and an energy range of 5000: the backward deltas are carried without the
