@@ -67,6 +67,15 @@ __device__ __forceinline__ int xcd_contiguous_block(int b, int nb) {
     return x * per + (x < extra ? x : extra) + r;
 }
 
+// ---- wave-level LDS order -----------------------------------------------------
+// Orders LDS accesses of the lanes of one wave: the hardware executes a wave's
+// LDS instructions in order, the fences keep the compiler from moving them.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- per-component force / torque clip -------------------------------------
 // v > c -> c, v < -c -> -c, anything else (including NaN) unchanged: the
 // masked assignments of ForceEvaluator.py:125-131.  c <= 0 disables the clip.

@@ -60,14 +60,6 @@ __device__ __forceinline__ float quad_sum(float v) {
     return v;
 }
 
-// Orders LDS accesses of the lanes of one wave: the hardware executes a wave's
-// LDS instructions in order, the fences keep the compiler from moving them.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ float sel4(int q, float v0, float v1, float v2, float v3) {
     return q == 0 ? v0 : q == 1 ? v1 : q == 2 ? v2 : v3;
 }

@@ -131,3 +131,35 @@ def test_bead_nvt_temperatures_reach_kT(gpu):
     print(f"bead NVT: T_t {t0[0]:.3f} -> <T_t>/kT {mt:.4f}, T_r {t0[1]:.3f} -> <T_r>/kT {mr:.4f} "
           f"(std {np.std(Tt[100:]) / spec.kT:.3f}, {np.std(Tr[100:]) / spec.kT:.3f})")
     assert t0[0] > 1.2 and abs(mt - 1.0) < 0.05 and abs(mr - 1.0) < 0.05
+
+
+@pytest.mark.parametrize("n_beads", [1, 5, 64, 65, 152, 256])
+def test_bead_cull_keeps_every_pair_in_reach(gpu, n_beads):
+    """Bead tables of every lane-remainder, off the body's centre and of unequal sides, at centre
+    distances from overlapping to out of reach and with quaternions of norm other than one (the
+    rotation formula then scales the body): the culled sums equal the oracle's over all bead pairs."""
+    from nepx import _lib, label
+    rng = np.random.default_rng(n_beads)
+    beads = (rng.uniform(-1.0, 1.0, (n_beads, 3)) * [2.2, 1.1, 0.4] + [0.6, -0.3, 0.2]).astype(np.float32)
+    P = 600
+    q = rng.normal(size=(2 * P, 4))
+    q *= (rng.uniform(0.8, 1.25, 2 * P) / np.linalg.norm(q, axis=1))[:, None]
+    q = q.astype(np.float32)
+    d = rng.normal(size=(P, 3))
+    t = (d / np.linalg.norm(d, axis=1)[:, None] * np.linspace(0.2, 9.0, P)[:, None]).astype(np.float32)
+    pot = label.BeadPotential(beads=beads, device=gpu)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    qf, pi, pj = dev(q), dev(np.arange(P, dtype=np.int32)), dev(np.arange(P, 2 * P, dtype=np.int32))
+    pt = dev(np.concatenate([t, np.zeros((P, 1), np.float32)], 1))
+    out = torch.full((P * 12,), float("nan"), device=gpu)
+    n_dev = torch.tensor([P], dtype=torch.int32, device=gpu)
+    pot.pair_forces(_lib.ptr(qf), _lib.ptr(pi), _lib.ptr(pj), _lib.ptr(pt), _lib.ptr(n_dev), P, _lib.ptr(out))
+    got = out.view(P, 12).cpu().numpy()
+    X = np.concatenate([np.zeros((P, 3)), t.astype(np.float64)])
+    pairs = np.stack([np.arange(P), np.arange(P, 2 * P)], 1)
+    r = O.bead_pair_forces(X, q.astype(np.float64), pairs, beads.astype(np.float64), 1e3)
+    assert np.count_nonzero(r["E"]) >= (3 if n_beads == 1 else 50)
+    assert np.array_equal(got[:, 3] != 0.0, r["E"] > 0.0) or np.abs(got[:, 3] - r["E"]).max() < 1e-9
+    for a, b, tol in ((got[:, 3], r["E"], 1e-5), (got[:, 0:3], r["F"], 1e-4), (got[:, 4:7], r["Ti"], 1e-4),
+                      (got[:, 8:11], r["Tj"], 1e-4)):
+        assert np.abs(a - b).max() <= tol * np.abs(b).max()
