@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+#include <type_traits>
+
 #include "../../include/nepx.h"
 
 namespace nepx {
@@ -39,6 +41,14 @@ nepx_tuning tuning();        // current values with defaults filled in
 int device_cus();            // compute units of the current device
 
 // ---- compile-time helpers --------------------------------------------------
+// fn(integral_constant<int, 0>), ..., fn(integral_constant<int, COUNT - 1>)
+template <int COUNT, int I = 0, class Fn>
+__device__ __forceinline__ void static_for(Fn&& fn) {
+    if constexpr (I < COUNT) {
+        fn(std::integral_constant<int, I>{});
+        static_for<COUNT, I + 1>(fn);
+    }
+}
 constexpr double csqrt(double x) {
     double r = x > 1.0 ? x : 1.0;
     for (int i = 0; i < 64; ++i) r = 0.5 * (r + x / r);

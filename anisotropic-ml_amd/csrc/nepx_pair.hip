@@ -250,14 +250,6 @@ struct SpreadNet {
 // Operand chunks in flight per wave: the fewer products a chunk feeds, the further ahead it is read.
 constexpr int spread_depth(int nt) { return nt >= 4 ? 3 : nt == 2 ? 4 : 6; }
 
-template <int COUNT, int I = 0, class Fn>
-__device__ __forceinline__ void static_for(Fn&& fn) {
-    if constexpr (I < COUNT) {
-        fn(std::integral_constant<int, I>{});
-        static_for<COUNT, I + 1>(fn);
-    }
-}
-
 template <class N, int ACT, int NT>
 __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float en_min, float scale, int D,
                                             const float* __restrict__ G, int P, int tile0, float* __restrict__ E,
@@ -659,19 +651,27 @@ static void launch_desc_fwd(const nepx_pair_model& m, const float* qf, const int
 }
 
 template <class T>
-static void launch_adjoint(const nepx_pair_model& m, const float* qf, const int32_t* pair_i, const int32_t* pair_j,
-                           const float* pair_t, const int32_t* np_dev, int64_t maxp, const float* dEdG,
-                           const float* E, float clip, float* out, void* stream) {
-    if constexpr (!T::ONE_PASS) {
-        if (by_passes<T>(maxp)) {
-            hipLaunchKernelGGL(k_adjoint_passes<T>, dim3(pass_grid(maxp)), dim3(64 * pass_waves<T>()), 0,
-                               as_stream(stream), m, (const float4*)qf, pair_i, pair_j, (const float4*)pair_t,
-                               np_dev, maxp, dEdG, E, clip, out);
-            return;
+static int launch_adjoint(const nepx_pair_model& m, const float* qf, const int32_t* pair_i, const int32_t* pair_j,
+                          const float* pair_t, const int32_t* np_dev, int64_t maxp, const float* dEdG,
+                          const float* E, float clip, float* out, void* stream) {
+    if constexpr (adjoint_on_quads<T>()) {
+        return launch_adjoint_quad<T>(m, (int)(device_cus() * (int64_t)tuning().pair_blocks_per_cu), qf, pair_i,
+                                      pair_j, pair_t, np_dev, maxp, dEdG, E, clip, out, stream);
+    } else {
+        if constexpr (!T::ONE_PASS) {
+            if (by_passes<T>(maxp)) {
+                hipLaunchKernelGGL(k_adjoint_passes<T>, dim3(pass_grid(maxp)), dim3(64 * pass_waves<T>()), 0,
+                                   as_stream(stream), m, (const float4*)qf, pair_i, pair_j, (const float4*)pair_t,
+                                   np_dev, maxp, dEdG, E, clip, out);
+                NEPX_LAUNCH_CHECK();
+                return NEPX_OK;
+            }
         }
+        hipLaunchKernelGGL(k_adjoint<T>, dim3(grid_for(maxp, kBlock)), dim3(kBlock), 0, as_stream(stream), m,
+                           (const float4*)qf, pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, dEdG, E, clip, out);
+        NEPX_LAUNCH_CHECK();
+        return NEPX_OK;
     }
-    hipLaunchKernelGGL(k_adjoint<T>, dim3(grid_for(maxp, kBlock)), dim3(kBlock), 0, as_stream(stream), m,
-                       (const float4*)qf, pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, dEdG, E, clip, out);
 }
 
 static bool desc_supported(const nepx_pair_model* m) {
@@ -972,9 +972,7 @@ extern "C" int nepx_descriptor_adjoint(const nepx_pair_model* m, const float* qf
     if (maxp <= 0) return NEPX_OK;
 #define X(ns, a, b, c, T)                                                                            \
     if (m->n_sites == ns && m->nrad == a && m->nang == b && m->lmax == c) {                         \
-        launch_adjoint<T>(*m, qf, pair_i, pair_j, pair_t, np_dev, maxp, dEdG, E, clip, out, stream);  \
-        NEPX_LAUNCH_CHECK();                                                                         \
-        return NEPX_OK;                                                                              \
+        return launch_adjoint<T>(*m, qf, pair_i, pair_j, pair_t, np_dev, maxp, dEdG, E, clip, out, stream); \
     }
     NEPX_DESC_CASES(X)
 #undef X

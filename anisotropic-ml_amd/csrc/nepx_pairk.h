@@ -203,6 +203,18 @@ struct QuadCfg {
     static constexpr int BLOCK = 256 * WAVES_PER_SIMD;
 };
 
+// Shapes whose adjoint runs four lanes per pair (nepx_quad_adjoint.h): those without a fused kernel.  The
+// shapes with one keep k_adjoint, whose results equal the one-lane fused kernel's bit for bit.
+template <class Cfg>
+constexpr bool adjoint_on_quads() {
+    return std::is_same<Cfg, CfgCubeV2>::value || std::is_same<Cfg, CfgThV1>::value ||
+           std::is_same<Cfg, CfgCubeV2L10>::value || std::is_same<Cfg, CfgThV1L10>::value;
+}
+template <class Cfg>
+int launch_adjoint_quad(const nepx_pair_model& m, int max_blocks, const float* qf, const int32_t* pair_i,
+                        const int32_t* pair_j, const float* pair_t, const int32_t* np_dev, int64_t maxp,
+                        const float* dEdG, const float* E, float clip, float* out, void* stream);
+
 // Fused descriptor -> network -> adjoint with four lanes per pair and the site
 // sums on matrix cores (nepx_quad.hip), on at most max_blocks blocks.  Returns
 // NEPX_EUNSUP for shapes it does not cover.

@@ -1,0 +1,379 @@
+// Descriptor adjoint from dE/dG in memory with the per-pair contractions on matrix cores: four lanes
+// per pair, 16 pairs per tile, as in the fused kernel (nepx_quad.h has the layout of the
+// v_mfma_f32_4x4x1_16b_f32 products), for the shapes whose network has no fused kernel.
+//
+// The one-lane-per-pair adjoint (k_adjoint) cuts the l range into passes that fit one lane's registers
+// and evaluates the sites' geometry, radial functions and harmonics again for every pass, forward and
+// back: eight passes for hypers 10 10 10.  Here the harmonics are cut by m instead of l: the columns
+// m of Q_l^m follow from Q_m^m by a recurrence in l alone, and the gradient of column m needs only
+// columns m and m + 1, so a group of m repeats next to nothing of another group's harmonics.  Each
+// group of a tile runs on its own wave (hypers 10 10 10: m = {0, 1}, {2, 5}, {3, 4} and {6..10}, 30 of
+// the 120 harmonics each, two waves per SIMD; hypers 10 8 4: all on one wave), and the groups' per-body
+// sums meet in LDS in a fixed order.  The bound is VALU issue (site geometry, radial functions and the
+// per-site gradient sums) and, with two waves per SIMD, the waits of its chains.  8 (12) sites, hypers
+// 10 10 10: 241 pairs 45 -> 13 us (61 -> 15), 20,000 pairs 92 -> 62 us (128 -> 68), 100,001 pairs
+// 310 -> 233 us (419 -> 262); hypers 10 8 4: 241 pairs 15 -> 13 us (20 -> 13), 100,001 pairs 52 -> 40 us
+// (72 -> 50).
+#pragma once
+#include "nepx_quad.h"
+
+namespace nepx {
+
+// Harmonics of the m in the bit set MASK, max(m, 1) <= l <= LMAX: slots ordered by m, part, l.
+template <int LMAX_, unsigned MASK>
+struct MSet {
+    static constexpr int LMAX = LMAX_;
+    __host__ __device__ static constexpr bool has(int m) { return (MASK >> m) & 1u; }
+    // columns of Q the sums and the gradient read: m and m + 1
+    __host__ __device__ static constexpr bool column(int m) { return m <= LMAX && (has(m) || (m > 0 && has(m - 1))); }
+    __host__ __device__ static constexpr int first_l(int m) { return m > 1 ? m : 1; }
+    __host__ __device__ static constexpr int rows(int m) { return LMAX - first_l(m) + 1; }
+    __host__ __device__ static constexpr int off(int m) {
+        int o = 0;
+        for (int k = 0; k < m; ++k) o += has(k) ? rows(k) * (k ? 2 : 1) : 0;
+        return o;
+    }
+    static constexpr int N = off(LMAX + 1);
+    __host__ __device__ static constexpr int slot(int l, int m, int part) {
+        return off(m) + part * rows(m) + l - first_l(m);
+    }
+    __host__ __device__ static constexpr int m_of(int s) {
+        int m = 0;
+        while (s >= off(m + 1)) ++m;
+        return m;
+    }
+    __host__ __device__ static constexpr int l_of(int s) {
+        const int m = m_of(s);
+        return first_l(m) + (s - off(m)) % rows(m);
+    }
+    // 2 K_lm^2 and the entry of l within dE/dg_ang[n] of slot s; zero and 0 past the last slot
+    __host__ __device__ static constexpr float two_k2(int s) {
+        return s < N ? 2.f * K2Tab<LMAX>{}(l_of(s), m_of(s)) : 0.f;
+    }
+    __host__ __device__ static constexpr int row_of(int s) { return s < N ? l_of(s) - 1 : 0; }
+};
+
+// The columns of Q_l^m a set reads, and C_m, S_m (nepx_desc.h's Harm, column by column).
+template <class MS>
+struct HarmM {
+    static constexpr int L = MS::LMAX;
+    float Q[L + 1][L + 1];  // [m][l], the set's columns
+    float C[L + 1], S[L + 1];
+    __device__ __forceinline__ float q(int l, int m) const { return Q[m][l]; }
+    __device__ __forceinline__ float z(int l, int m, int part) const {
+        return m == 0 ? q(l, 0) : q(l, m) * (part ? S[m] : C[m]);
+    }
+    __device__ __forceinline__ void eval(float x, float y, float zz) {
+        float qmm = 1.f;
+#pragma unroll
+        for (int m = 0; m <= L; ++m) {
+            if (m > 0) qmm *= -(2.f * m - 1.f);
+            if (MS::column(m)) {
+                Q[m][m] = qmm;
+                if (m < L) Q[m][m + 1] = (2.f * m + 1.f) * zz * qmm;
+#pragma unroll
+                for (int l = m + 2; l <= L; ++l) {
+                    const float a = (2.f * l - 1.f) / (float)(l - m);
+                    const float b = (float)(l + m - 1) / (float)(l - m);
+                    Q[m][l] = a * zz * Q[m][l - 1] - b * Q[m][l - 2];
+                }
+            }
+        }
+        C[0] = 1.f;
+        S[0] = 0.f;
+#pragma unroll
+        for (int m = 1; m <= L; ++m) {  // the powers past the set's last m are never read
+            C[m] = x * C[m - 1] - y * S[m - 1];
+            S[m] = x * S[m - 1] + y * C[m - 1];
+        }
+    }
+};
+
+// The part of angular_site_grad (nepx_desc.h) that the m of a set contribute.
+template <class MS, class CD>
+__device__ __forceinline__ void angular_site_grad_m(const HarmM<MS>& h, float ux, float uy, CD&& cd, float& dEdrho,
+                                                    float& gx, float& gy, float& gz) {
+    float E1 = 0.f, Gz = 0.f, X1 = 0.f, Y1 = 0.f;
+#pragma unroll
+    for (int mm = 0; mm <= MS::LMAX; ++mm) {
+        if (!MS::has(mm)) continue;
+        float U[2] = {0.f, 0.f}, V[2] = {0.f, 0.f}, W[2] = {0.f, 0.f}, Dq[2] = {0.f, 0.f};
+#pragma unroll
+        for (int l = MS::first_l(mm); l <= MS::LMAX; ++l) {
+            const float ql = h.q(l, mm);
+            const float qa = (mm + 1 <= l - 1) ? h.q(l - 1, mm + 1) : 0.f;
+            const float qc = (mm <= l - 1) ? (float)(l + mm) * h.q(l - 1, mm) : 0.f;
+#pragma unroll
+            for (int part = 0; part < (mm ? 2 : 1); ++part) {
+                float c, d;
+                cd(MS::slot(l, mm, part), c, d);
+                Dq[part] += d * ql;
+                if (mm + 1 <= l - 1) U[part] += qa * c;
+                if (mm <= l - 1) V[part] += qc * c;
+                if (mm >= 1) W[part] += ql * c;
+            }
+        }
+        dEdrho += mm == 0 ? Dq[0] : h.C[mm] * Dq[0] + h.S[mm] * Dq[1];
+        if (mm == 0) {
+            E1 += U[0];
+            Gz += V[0];
+        } else {
+            E1 += h.C[mm] * U[0] + h.S[mm] * U[1];
+            Gz += h.C[mm] * V[0] + h.S[mm] * V[1];
+            const float fm = (float)mm;
+            X1 += fm * (h.C[mm - 1] * W[0] + h.S[mm - 1] * W[1]);
+            Y1 += fm * (h.C[mm - 1] * W[1] - h.S[mm - 1] * W[0]);
+        }
+    }
+    gx = ux * E1 + X1;
+    gy = uy * E1 + Y1;
+    gz = Gz;
+}
+
+// Groups of m, one wave each; the radial terms go with one of them.
+template <int LMAX>
+struct MGroups {  // all m on one wave
+    static constexpr int COUNT = 1, RAD = 0;
+    template <int G>
+    using Set = MSet<LMAX, (2u << LMAX) - 1u>;
+};
+template <>
+struct MGroups<10> {  // 30 harmonics each
+    static constexpr int COUNT = 4, RAD = 2;
+    static constexpr unsigned MASK[4] = {0x003, 0x024, 0x018, 0x7c0};
+    template <int G>
+    using Set = MSet<10, MASK[G]>;
+};
+
+template <class Cfg>
+struct QuadAdj {
+    using MG = MGroups<Cfg::LMAX>;
+    static constexpr int NA = Cfg::NANG + 1, NC = (NA + 3) / 4, STEPS = Cfg::ND / 4, BLOCK = 64 * MG::COUNT;
+    static constexpr bool OK = Cfg::ND % 4 == 0;
+    template <int G>
+    static constexpr int chunks() { return (MG::template Set<G>::N + 3) / 4; }
+    template <int G = 0>
+    static constexpr int max_chunks() {
+        if constexpr (G + 1 < MG::COUNT) {
+            return chunks<G>() > max_chunks<G + 1>() ? chunks<G>() : max_chunks<G + 1>();
+        } else {
+            return chunks<G>();
+        }
+    }
+    // exchange floats per pair, TS / 4 odd (as QuadCfg::TS)
+    static constexpr int TS = (NC + max_chunks()) * 16 + 4;
+};
+
+// One tile's sums over its sites for the harmonics of MR (and the radial terms with RAD): dE/dr and
+// arm x dE/dr per body, the same in all four lanes of a pair.
+template <class Cfg, class MS, bool RAD>
+__device__ __forceinline__ void quad_adjoint_sums(const nepx_pair_model& m, const float4* stab, const PairIn& g,
+                                                  const float* grow, float* xp, int q, float (&sum)[12]) {
+    using Q = QuadAdj<Cfg>;
+    constexpr int NC = Q::NC, NA = Q::NA, LC = (MS::N + 3) / 4, LMAX = Cfg::LMAX;
+    constexpr int GA = Cfg::NRAD + 1;
+    const float inv_rn = 1.f / m.r_nep;
+    auto site = [&](int s, bool& bj) {  // this lane's site a = 4s + q
+        int a = 4 * s + q;
+        bj = a >= Cfg::NS;
+        // opaque: the compiler would keep every trip's geometry and harmonics from the forward for
+        // the adjoint, hundreds of registers
+        asm volatile("" : "+v"(a));
+        const float4 b = stab[a];
+        const Mat3 Rb = quat_matrix(bj ? g.qj.x : g.qi.x, bj ? g.qj.y : g.qi.y, bj ? g.qj.z : g.qi.z,
+                                    bj ? g.qj.w : g.qi.w);
+        return site_geo_b(Rb, b.x, b.y, b.z, (bj ? g.tx : 0.f) - g.cx, (bj ? g.ty : 0.f) - g.cy,
+                          (bj ? g.tz : 0.f) - g.cz, inv_rn);
+    };
+    // ---- forward: A[n][slot] ----
+    v4f Af[NC][LC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int d = 0; d < LC; ++d) Af[c][d] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = 0; s < Q::STEPS; ++s) {
+        bool bj;
+        const SiteGeo sg = site(s, bj);
+        float fv[4 * NC];
+#pragma unroll
+        for (int n = NA; n < 4 * NC; ++n) fv[n] = 0.f;
+        radial_values<Cfg::NANG>(sg.rho, 1.f, [&](int n, float f) { fv[n] = f; });
+        HarmM<MS> h;
+        h.eval(sg.ux, sg.uy, sg.uz);
+        wave_lds_order();
+#pragma unroll
+        for (int n = 0; n < 4 * NC; ++n) xp[16 * (n / 4) + 4 * (n % 4) + q] = fv[n];
+#pragma unroll
+        for (int mm = 0; mm <= LMAX; ++mm)
+#pragma unroll
+            for (int part = 0; part < (MS::has(mm) ? (mm ? 2 : 1) : 0); ++part)
+#pragma unroll
+                for (int l = MS::first_l(mm); l <= LMAX; ++l) {
+                    const int o = MS::slot(l, mm, part);
+                    xp[16 * (NC + o / 4) + 4 * (o % 4) + q] = h.z(l, mm, part);
+                }
+#pragma unroll
+        for (int o = MS::N; o < 4 * LC; ++o) xp[16 * (NC + o / 4) + 4 * (o % 4) + q] = 0.f;
+        wave_lds_order();
+        v4f xf[NC], xz[LC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) xf[c] = *reinterpret_cast<const v4f*>(xp + 16 * c + 4 * q);
+#pragma unroll
+        for (int d = 0; d < LC; ++d) xz[d] = *reinterpret_cast<const v4f*>(xp + 16 * (NC + d) + 4 * q);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int d = 0; d < LC; ++d)
+                    Af[c][d] = __builtin_amdgcn_mfma_f32_4x4x1f32(
+                        xf[c][k], xz[d][k], Af[c][d], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // ---- B = dE/dA = 2 K^2 dE/dg_ang[n][l] A: this lane's column of chunk d is slot 4d + q ----
+    static_for<LC>([&](auto dc) {
+        constexpr int d = decltype(dc)::value;
+        constexpr float w0 = MS::two_k2(4 * d), w1 = MS::two_k2(4 * d + 1), w2 = MS::two_k2(4 * d + 2),
+                        w3 = MS::two_k2(4 * d + 3);
+        constexpr int a0 = MS::row_of(4 * d), a1 = MS::row_of(4 * d + 1), a2 = MS::row_of(4 * d + 2),
+                      a3 = MS::row_of(4 * d + 3);
+        const float kw = sel4(q, w0, w1, w2, w3);
+        const float* row = grow + GA + (q == 0 ? a0 : q == 1 ? a1 : q == 2 ? a2 : a3);
+#pragma unroll
+        for (int n = 0; n < NA; ++n) Af[n / 4][d][n % 4] *= kw * row[n * LMAX];
+    });
+    float dGr[Cfg::NRAD + 1], ndGr[Cfg::NRAD + 1];
+    float dGr_hi = 0.f;
+    if constexpr (RAD) {
+#pragma unroll
+        for (int n = 0; n <= Cfg::NRAD; ++n) {
+            dGr[n] = grow[n];
+            ndGr[n] = (float)n * dGr[n];
+            if (n >= NA) dGr_hi += dGr[n];
+        }
+    }
+    // ---- adjoint ----
+    float ig_x = 0.f, ig_y = 0.f, ig_z = 0.f, it_x = 0.f, it_y = 0.f, it_z = 0.f;
+    float jg_x = 0.f, jg_y = 0.f, jg_z = 0.f, jt_x = 0.f, jt_y = 0.f, jt_z = 0.f;
+#pragma unroll 1
+    for (int s = 0; s < Q::STEPS; ++s) {
+        bool bj;
+        const SiteGeo sg = site(s, bj);
+        float fa[NA], da[NA];
+        float dEdrho = 0.f;
+        if constexpr (RAD) {
+            dEdrho = radial_adjoint<Cfg::NRAD, NA>(sg.rho, dGr, ndGr, dGr_hi, fa, da);
+        } else {
+            radial_derivs<Cfg::NANG>(sg.rho, [&](int n, float f, float df) {
+                fa[n] = f;
+                da[n] = df;
+            });
+        }
+        v4f cc[LC], dd[LC];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < NA; ++n)
+#pragma unroll
+            for (int d = 0; d < LC; ++d) {
+                const float b = Af[n / 4][d][n % 4];
+                const v4f z4 = {0.f, 0.f, 0.f, 0.f};
+                cc[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(b, fa[n], n == 0 ? z4 : cc[d], 0, 0, 0);
+                dd[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(b, da[n], n == 0 ? z4 : dd[d], 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        HarmM<MS> h;
+        h.eval(sg.ux, sg.uy, sg.uz);
+        float gx, gy, gz;
+        angular_site_grad_m<MS>(
+            h, sg.ux, sg.uy,
+            [&](int o, float& c, float& dv) {
+                c = cc[o / 4][o % 4];
+                dv = dd[o / 4][o % 4];
+            },
+            dEdrho, gx, gy, gz);
+        float ex, ey, ez;
+        site_dEdr(sg, dEdrho, inv_rn, gx, gy, gz, ex, ey, ez);
+        const float tx = sg.ay * ez - sg.az * ey, ty = sg.az * ex - sg.ax * ez, tz = sg.ax * ey - sg.ay * ex;
+        const float wj = bj ? 1.f : 0.f, wi = 1.f - wj;
+        ig_x += wi * ex; ig_y += wi * ey; ig_z += wi * ez;
+        it_x += wi * tx; it_y += wi * ty; it_z += wi * tz;
+        jg_x += wj * ex; jg_y += wj * ey; jg_z += wj * ez;
+        jt_x += wj * tx; jt_y += wj * ty; jt_z += wj * tz;
+    }
+    sum[0] = quad_sum(ig_x); sum[1] = quad_sum(ig_y); sum[2] = quad_sum(ig_z);
+    sum[3] = quad_sum(it_x); sum[4] = quad_sum(it_y); sum[5] = quad_sum(it_z);
+    sum[6] = quad_sum(jg_x); sum[7] = quad_sum(jg_y); sum[8] = quad_sum(jg_z);
+    sum[9] = quad_sum(jt_x); sum[10] = quad_sum(jt_y); sum[11] = quad_sum(jt_z);
+}
+
+template <class Cfg>
+__global__ __launch_bounds__((QuadAdj<Cfg>::BLOCK)) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adjoint_quad(
+    nepx_pair_model m, const float4* __restrict__ qf, const int32_t* __restrict__ pi, const int32_t* __restrict__ pj,
+    const float4* __restrict__ pt, const int32_t* __restrict__ np_dev, int64_t maxp,
+    const float* __restrict__ dEdG, const float* __restrict__ E, float clip, float* __restrict__ out) {
+    using Q = QuadAdj<Cfg>;
+    using MG = typename Q::MG;
+    constexpr int PW = 16, D = Cfg::D, COUNT = MG::COUNT;
+    __shared__ __attribute__((aligned(16))) float xch[COUNT][PW * Q::TS];
+    __shared__ float rows[PW * D];
+    __shared__ float part[COUNT][12][PW];
+    __shared__ float4 stab[Cfg::ND];
+    if (threadIdx.x < Cfg::ND) {
+        const int k = threadIdx.x % Cfg::NS;
+        stab[threadIdx.x] = make_float4(m.sites[3 * k], m.sites[3 * k + 1], m.sites[3 * k + 2], 0.f);
+    }
+    const int P = n_pairs(np_dev, maxp);
+    const int lane = threadIdx.x & 63, q = lane & 3, slot = lane >> 2;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float* const xp = xch[wave] + slot * Q::TS;
+    for (int base = blockIdx.x * PW; base < P; base += gridDim.x * PW) {  // uniform over the block
+        const int idx = base + slot;
+        const bool valid = idx < P;
+        float4 qi = make_float4(1.f, 0.f, 0.f, 0.f), qj = qi, t = make_float4(1.f, 0.f, 0.f, 0.f);
+        if (valid) load_pair(qf, pi, pj, pt, idx, qi, qj, t);
+        // the tile's dE/dG rows are contiguous
+        const int have = (P - base < PW ? P - base : PW) * D;
+        for (int k = threadIdx.x; k < PW * D; k += Q::BLOCK) rows[k] = k < have ? dEdG[(size_t)base * D + k] : 0.f;
+        const PairIn g = pair_in<Cfg>(m, qi, qj, t.x, t.y, t.z);
+        __syncthreads();
+        const float* grow = rows + slot * D;
+        float sum[12];
+        if constexpr (COUNT == 1) {
+            quad_adjoint_sums<Cfg, typename MG::template Set<0>, true>(m, stab, g, grow, xp, q, sum);
+        } else {
+            static_for<COUNT>([&](auto gc) {
+                constexpr int G = decltype(gc)::value;
+                if (wave == G)
+                    quad_adjoint_sums<Cfg, typename MG::template Set<G>, G == MG::RAD>(m, stab, g, grow, xp, q, sum);
+            });
+            if (q == 0) {
+#pragma unroll
+                for (int c = 0; c < 12; ++c) part[wave][c][slot] = sum[c];
+            }
+        }
+        __syncthreads();  // the groups' sums are there, and every read of the rows is done
+        if (wave == 0 && q == 0 && valid) {
+            if constexpr (COUNT > 1) {
+#pragma unroll
+                for (int c = 0; c < 12; ++c) {
+                    sum[c] = part[0][c][slot];
+#pragma unroll
+                    for (int w = 1; w < COUNT; ++w) sum[c] += part[w][c][slot];
+                }
+            }
+            AdjAcc acc;
+            acc.G0x = sum[0]; acc.G0y = sum[1]; acc.G0z = sum[2];
+            acc.T0x = sum[3]; acc.T0y = sum[4]; acc.T0z = sum[5];
+            acc.G1x = sum[6]; acc.G1y = sum[7]; acc.G1z = sum[8];
+            acc.T1x = sum[9]; acc.T1y = sum[10]; acc.T1z = sum[11];
+            acc.A0x = g.six; acc.A0y = g.siy; acc.A0z = g.siz;
+            acc.A1x = g.sjx; acc.A1y = g.sjy; acc.A1z = g.sjz;
+            store_out(out, idx, adj_finish<Cfg>(acc), E ? E[idx] : 0.f, clip);
+        }
+        // the next tile's sums are written after its first barrier, which wave 0 reaches past these reads
+    }
+}
+
+}  // namespace nepx

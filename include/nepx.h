@@ -184,7 +184,7 @@ int nepx_net_pack_lowp(int32_t precision, int32_t d_in, int32_t width, int32_t n
 
 /* ---- descriptor, energy network, adjoint ------------------------------- */
 /* P = min(*n_pairs_dev, max_pairs) is read on the device; max_pairs sizes the launch.  Up to about
- * 2 x 64 pairs per CU (descriptor, adjoint of multi-pass shapes) the work of one pair is spread over
+ * 2 x 64 pairs per CU (descriptor of multi-pass shapes) the work of one pair is spread over
  * several waves, and the FP32 network spreads its layers over a block's waves (up to 4 x 16 pairs per
  * CU, or any number for networks too wide for LDS); the results are the same bit for bit. */
 /* G (P x D, f32) of compacted pairs.  Replaces pos_to_pts + pts_to_nep_descriptors

@@ -192,6 +192,37 @@ def test_adjoint_matches_oracle(gpu, shape_name, hyp):
     assert max(eF, eTi, eTj) < 1e-4
 
 
+@pytest.mark.parametrize("n_pairs", [1, 15, 17, 1025])
+@pytest.mark.parametrize("shape_name,hyp", [("cube_v2", (10, 8, 4)), ("th_v1", (10, 8, 4)),
+                                            ("cube_v2", (10, 10, 10)), ("th_v1", (10, 10, 10))])
+def test_quad_adjoint_tile_edges(gpu, shape_name, hyp, n_pairs):
+    """The four-lane adjoint takes 16 pairs per tile: tiles with one pair, one short, one over and a ragged
+    last one, forces and torques against the FP64 oracle, and a device count below the capacity."""
+    import nepx
+    from nepx import ops
+    shape, (q, i, j, t), T = _inputs(gpu, shape_name, n_pairs=n_pairs, seed=15)
+    model = nepx.make_pair_model(shape, hyp)
+    D = nepx.n_descriptor(*hyp)
+    dG = np.random.default_rng(16).standard_normal((n_pairs, D)).astype(np.float32)
+    E = torch.linspace(-2.0, 2.0, n_pairs, device=gpu)
+    out = ops.descriptor_adjoint(model, T["qf"], T["pi"], T["pj"], T["pt"], torch.from_numpy(dG).to(gpu), E=E)
+    clouds = oracle_clouds(q, i, j, t, shape.sites)
+    gp = O.descriptor_grad(clouds, dG.astype(np.float64), shape.nep_cutoff, *hyp)
+    Ns = shape.n_sites
+    arm_j = clouds[:, Ns:] - t.astype(np.float64)[:, None, :]
+    want = np.concatenate([-gp[:, :Ns].sum(1), np.cross(clouds[:, :Ns], -gp[:, :Ns]).sum(1),
+                           np.cross(arm_j, -gp[:, Ns:]).sum(1)], 1)
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:, 3], E.cpu().numpy())
+    for a, b in ((0, 0), (4, 3), (8, 6)):
+        assert normwise_rel(got[:, a:a + 3], want[:, b:b + 3]) < 1e-4
+    if n_pairs > 16:   # the device count, not the capacity, bounds the rows
+        n_dev = torch.tensor([n_pairs - 3], dtype=torch.int32, device=gpu)
+        part = ops.descriptor_adjoint(model, T["qf"], T["pi"], T["pj"], T["pt"], torch.from_numpy(dG).to(gpu), E=E,
+                                      n_dev=n_dev)
+        assert torch.equal(part[:n_pairs - 3], out[:n_pairs - 3])
+
+
 @pytest.mark.parametrize("shape_name,hyp", CASES)
 def test_pass_kernels_equal_pair_kernels(gpu, shape_name, hyp):
     """Few pairs of a multi-pass shape run their l-range passes on separate waves (descriptor and
