@@ -341,44 +341,6 @@ struct PairSites {  // the 2 Ns sites of one pair, bodies i (0) and j (1), weigh
     }
 };
 
-struct CloudSites {  // nd points of a site cloud (xyz interleaved), optional per-point weights
-    const float* __restrict__ pts;
-    const float* __restrict__ w;
-    int nd;
-    float cx, cy, cz, inv_rn;
-    __device__ __forceinline__ CloudSites(const float* pts_, const float* w_, int nd_, float inv_rn_)
-        : pts(pts_), w(w_), nd(nd_), inv_rn(inv_rn_) {
-        float sx = 0.f, sy = 0.f, sz = 0.f;
-        for (int a = 0; a < nd; ++a) {
-            sx += pts[3 * a];
-            sy += pts[3 * a + 1];
-            sz += pts[3 * a + 2];
-        }
-        const float inv = 1.f / (float)nd;
-        cx = sx * inv;
-        cy = sy * inv;
-        cz = sz * inv;
-    }
-    template <class S, class B>
-    __device__ __forceinline__ void visit(S&& site, B&& body_done) const {
-#pragma unroll 1
-        for (int a = 0; a < nd; ++a) {
-            SiteGeo s;
-            s.ax = s.ay = s.az = 0.f;
-            const float rx = pts[3 * a] - cx, ry = pts[3 * a + 1] - cy, rz = pts[3 * a + 2] - cz;
-            const float r2 = rx * rx + ry * ry + rz * rz;
-            s.ir = __builtin_amdgcn_rsqf(r2);
-            s.r = r2 * s.ir;
-            s.ux = rx * s.ir;
-            s.uy = ry * s.ir;
-            s.uz = rz * s.ir;
-            s.rho = s.r * inv_rn;
-            site(s, w ? w[a] : 1.f);
-        }
-        body_done(0);
-    }
-};
-
 // Forward accumulators over the l of range LR: A[n][lm - LR::OFF] = sum_a w_a f_n(a) Z_lm(u_a),
 // and (RAD) g_rad[n] = sum_a w_a f_n(a).
 template <class Cfg, class LR, bool RAD, class Sites>

@@ -6,7 +6,7 @@
 
 namespace nepx {
 
-// Descriptor row of one pair (or cloud), one pass over the sites per l range.
+// Descriptor row of one pair, one pass over the sites per l range.
 template <class Cfg, class Sites, class Row>
 __device__ __forceinline__ void desc_forward_sites(const Sites& sites, Row&& G) {
     float grad[Cfg::NRAD + 1];
@@ -1116,32 +1116,6 @@ extern "C" int nepx_fd_forces(const float* E_rows, int64_t P, float dx, float dt
     return NEPX_OK;
 }
 
-// ---------------------------------------------------------------------------
-// Descriptors of arbitrary site clouds (training-set featurisation,
-// 05/NEP.py:171-219 get_g_fast and 04/Processors.py:48-88): one cloud per
-// lane, sites relative to the cloud centroid, optional per-site weights.
-template <class Cfg>
-__global__ __launch_bounds__(kBlock) void k_cloud_desc(const float* __restrict__ clouds, int64_t P, int nd,
-                                                       const float* __restrict__ w, float r_nep,
-                                                       float* __restrict__ G) {
-    for (int64_t idx = blockIdx.x * (int64_t)kBlock + threadIdx.x; idx < P; idx += (int64_t)gridDim.x * kBlock) {
-        const CloudSites sites(clouds + idx * 3 * (int64_t)nd, w, nd, 1.f / r_nep);
-        if constexpr (Cfg::ONE_PASS) {
-            float Gr[Cfg::D];
-            desc_forward_sites<Cfg>(sites, Gr);
-            store_row<Cfg>(G + idx * Cfg::D, Gr);
-        } else {
-            desc_forward_sites<Cfg>(sites, G + idx * Cfg::D);
-        }
-    }
-}
-
-#define NEPX_CLOUD_CASES(X)     \
-    X(11, 6, 4)                 \
-    X(10, 8, 4)                 \
-    X(17, 6, 6)                 \
-    X(10, 10, 10)
-
 extern "C" int nepx_cloud_descriptor(const float* clouds, int64_t n_clouds, int32_t n_sites, const float* site_w,
                                      int32_t nrad, int32_t nang, int32_t lmax, float r_nep, float* G,
                                      void* stream) {
@@ -1150,14 +1124,10 @@ extern "C" int nepx_cloud_descriptor(const float* clouds, int64_t n_clouds, int3
     NEPX_REQUIRE(r_nep > 0.f, NEPX_EINVAL, "r_nep must be positive");
     if (n_clouds == 0) return NEPX_OK;
     NEPX_REQUIRE(clouds && G, NEPX_EINVAL, "null buffer");
-    const int grid = grid_for(n_clouds, kBlock);
-#define X(a, b, c)                                                                                     \
-    if (nrad == a && nang == b && lmax == c) {                                                         \
-        hipLaunchKernelGGL((k_cloud_desc<DescCfg<1, a, b, c>>), dim3(grid), dim3(kBlock), 0, as_stream(stream), \
-                           clouds, n_clouds, (int)n_sites, site_w, r_nep, G);                           \
-        NEPX_LAUNCH_CHECK();                                                                           \
-        return NEPX_OK;                                                                                \
-    }
+#define X(a, b, c)                                                                                       \
+    if (nrad == a && nang == b && lmax == c)                                                             \
+        return launch_cloud_quad<DescCfg<1, a, b, c>>(clouds, n_clouds, (int)n_sites, site_w, r_nep, G,  \
+                                                      stream);
     NEPX_CLOUD_CASES(X)
 #undef X
     set_error("no cloud descriptor kernel for hypers (%d, %d, %d)", nrad, nang, lmax);

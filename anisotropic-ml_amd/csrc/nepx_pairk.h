@@ -215,6 +215,18 @@ int launch_adjoint_quad(const nepx_pair_model& m, int max_blocks, const float* q
                         const int32_t* pair_j, const float* pair_t, const int32_t* np_dev, int64_t maxp,
                         const float* dEdG, const float* E, float clip, float* out, void* stream);
 
+// Hypers with a cloud descriptor kernel.
+#define NEPX_CLOUD_CASES(X)     \
+    X(11, 6, 4)                 \
+    X(10, 8, 4)                 \
+    X(17, 6, 6)                 \
+    X(10, 10, 10)
+
+// Descriptors of site clouds (nepx_quad_cloud.h); Cfg's site count is not used.
+template <class Cfg>
+int launch_cloud_quad(const float* clouds, int64_t n_clouds, int n_sites, const float* site_w, float r_nep,
+                      float* G, void* stream);
+
 // Fused descriptor -> network -> adjoint with four lanes per pair and the site
 // sums on matrix cores (nepx_quad.hip), on at most max_blocks blocks.  Returns
 // NEPX_EUNSUP for shapes it does not cover.

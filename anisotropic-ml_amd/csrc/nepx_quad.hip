@@ -1,9 +1,11 @@
-// Four-lanes-per-pair fused kernel (nepx_quad.h), adjoint (nepx_quad_adjoint.h) and their launchers.  Built in
+// Four-lanes-per-pair fused kernel (nepx_quad.h), adjoint (nepx_quad_adjoint.h) and cloud
+// descriptor (nepx_quad_cloud.h), and their launchers.  Built in
 // its own translation unit so that its matrix-core accumulators can be kept in
 // VGPRs (-mllvm -amdgpu-mfma-vgpr-form), next to the VALU code that reads them.
 #include "nepx_pairk.h"
 #include "nepx_quad.h"
 #include "nepx_quad_adjoint.h"
+#include "nepx_quad_cloud.h"
 
 namespace nepx {
 
@@ -83,5 +85,26 @@ NEPX_QUAD_ADJOINT(CfgThV1)
 NEPX_QUAD_ADJOINT(CfgCubeV2L10)
 NEPX_QUAD_ADJOINT(CfgThV1L10)
 #undef NEPX_QUAD_ADJOINT
+
+template <class Cfg>
+int launch_cloud_quad(const float* clouds, int64_t n_clouds, int n_sites, const float* site_w, float r_nep,
+                      float* G, void* stream) {
+    const int64_t tiles = (n_clouds + 15) / 16;
+    const int64_t resident = (int64_t)device_cus() * QuadCloud<Cfg>::BLOCKS_PER_CU;
+    const dim3 grid((unsigned)(tiles < resident ? tiles : resident)), block(QuadCloud<Cfg>::BLOCK);
+    if (n_sites <= QuadCloud<Cfg>::STAGED)
+        hipLaunchKernelGGL((k_cloud_quad<Cfg, true>), grid, block, 16 * 3 * n_sites * sizeof(float),
+                           as_stream(stream), clouds, n_clouds, n_sites, site_w, r_nep, G);
+    else
+        hipLaunchKernelGGL((k_cloud_quad<Cfg, false>), grid, block, 0, as_stream(stream), clouds, n_clouds, n_sites,
+                           site_w, r_nep, G);
+    NEPX_LAUNCH_CHECK();
+    return NEPX_OK;
+}
+#define NEPX_QUAD_CLOUD(a, b, c)                                                                               \
+    template int launch_cloud_quad<DescCfg<1, a, b, c>>(const float*, int64_t, int, const float*, float,      \
+                                                        float*, void*);
+NEPX_CLOUD_CASES(NEPX_QUAD_CLOUD)
+#undef NEPX_QUAD_CLOUD
 
 }  // namespace nepx

@@ -4,9 +4,7 @@
 //
 // The one-lane-per-pair adjoint (k_adjoint) cuts the l range into passes that fit one lane's registers
 // and evaluates the sites' geometry, radial functions and harmonics again for every pass, forward and
-// back: eight passes for hypers 10 10 10.  Here the harmonics are cut by m instead of l: the columns
-// m of Q_l^m follow from Q_m^m by a recurrence in l alone, and the gradient of column m needs only
-// columns m and m + 1, so a group of m repeats next to nothing of another group's harmonics.  Each
+// back: eight passes for hypers 10 10 10.  Here the harmonics are cut by m (nepx_msets.h).  Each
 // group of a tile runs on its own wave (hypers 10 10 10: m = {0, 1}, {2, 5}, {3, 4} and {6..10}, 30 of
 // the 120 harmonics each, two waves per SIMD; hypers 10 8 4: all on one wave), and the groups' per-body
 // sums meet in LDS in a fixed order.  The bound is VALU issue (site geometry, radial functions and the
@@ -15,79 +13,10 @@
 // 310 -> 233 us (419 -> 262); hypers 10 8 4: 241 pairs 15 -> 13 us (20 -> 13), 100,001 pairs 52 -> 40 us
 // (72 -> 50).
 #pragma once
+#include "nepx_msets.h"
 #include "nepx_quad.h"
 
 namespace nepx {
-
-// Harmonics of the m in the bit set MASK, max(m, 1) <= l <= LMAX: slots ordered by m, part, l.
-template <int LMAX_, unsigned MASK>
-struct MSet {
-    static constexpr int LMAX = LMAX_;
-    __host__ __device__ static constexpr bool has(int m) { return (MASK >> m) & 1u; }
-    // columns of Q the sums and the gradient read: m and m + 1
-    __host__ __device__ static constexpr bool column(int m) { return m <= LMAX && (has(m) || (m > 0 && has(m - 1))); }
-    __host__ __device__ static constexpr int first_l(int m) { return m > 1 ? m : 1; }
-    __host__ __device__ static constexpr int rows(int m) { return LMAX - first_l(m) + 1; }
-    __host__ __device__ static constexpr int off(int m) {
-        int o = 0;
-        for (int k = 0; k < m; ++k) o += has(k) ? rows(k) * (k ? 2 : 1) : 0;
-        return o;
-    }
-    static constexpr int N = off(LMAX + 1);
-    __host__ __device__ static constexpr int slot(int l, int m, int part) {
-        return off(m) + part * rows(m) + l - first_l(m);
-    }
-    __host__ __device__ static constexpr int m_of(int s) {
-        int m = 0;
-        while (s >= off(m + 1)) ++m;
-        return m;
-    }
-    __host__ __device__ static constexpr int l_of(int s) {
-        const int m = m_of(s);
-        return first_l(m) + (s - off(m)) % rows(m);
-    }
-    // 2 K_lm^2 and the entry of l within dE/dg_ang[n] of slot s; zero and 0 past the last slot
-    __host__ __device__ static constexpr float two_k2(int s) {
-        return s < N ? 2.f * K2Tab<LMAX>{}(l_of(s), m_of(s)) : 0.f;
-    }
-    __host__ __device__ static constexpr int row_of(int s) { return s < N ? l_of(s) - 1 : 0; }
-};
-
-// The columns of Q_l^m a set reads, and C_m, S_m (nepx_desc.h's Harm, column by column).
-template <class MS>
-struct HarmM {
-    static constexpr int L = MS::LMAX;
-    float Q[L + 1][L + 1];  // [m][l], the set's columns
-    float C[L + 1], S[L + 1];
-    __device__ __forceinline__ float q(int l, int m) const { return Q[m][l]; }
-    __device__ __forceinline__ float z(int l, int m, int part) const {
-        return m == 0 ? q(l, 0) : q(l, m) * (part ? S[m] : C[m]);
-    }
-    __device__ __forceinline__ void eval(float x, float y, float zz) {
-        float qmm = 1.f;
-#pragma unroll
-        for (int m = 0; m <= L; ++m) {
-            if (m > 0) qmm *= -(2.f * m - 1.f);
-            if (MS::column(m)) {
-                Q[m][m] = qmm;
-                if (m < L) Q[m][m + 1] = (2.f * m + 1.f) * zz * qmm;
-#pragma unroll
-                for (int l = m + 2; l <= L; ++l) {
-                    const float a = (2.f * l - 1.f) / (float)(l - m);
-                    const float b = (float)(l + m - 1) / (float)(l - m);
-                    Q[m][l] = a * zz * Q[m][l - 1] - b * Q[m][l - 2];
-                }
-            }
-        }
-        C[0] = 1.f;
-        S[0] = 0.f;
-#pragma unroll
-        for (int m = 1; m <= L; ++m) {  // the powers past the set's last m are never read
-            C[m] = x * C[m - 1] - y * S[m - 1];
-            S[m] = x * S[m - 1] + y * C[m - 1];
-        }
-    }
-};
 
 // The part of angular_site_grad (nepx_desc.h) that the m of a set contribute.
 template <class MS, class CD>
@@ -130,38 +59,13 @@ __device__ __forceinline__ void angular_site_grad_m(const HarmM<MS>& h, float ux
     gz = Gz;
 }
 
-// Groups of m, one wave each; the radial terms go with one of them.
-template <int LMAX>
-struct MGroups {  // all m on one wave
-    static constexpr int COUNT = 1, RAD = 0;
-    template <int G>
-    using Set = MSet<LMAX, (2u << LMAX) - 1u>;
-};
-template <>
-struct MGroups<10> {  // 30 harmonics each
-    static constexpr int COUNT = 4, RAD = 2;
-    static constexpr unsigned MASK[4] = {0x003, 0x024, 0x018, 0x7c0};
-    template <int G>
-    using Set = MSet<10, MASK[G]>;
-};
-
 template <class Cfg>
 struct QuadAdj {
     using MG = MGroups<Cfg::LMAX>;
     static constexpr int NA = Cfg::NANG + 1, NC = (NA + 3) / 4, STEPS = Cfg::ND / 4, BLOCK = 64 * MG::COUNT;
     static constexpr bool OK = Cfg::ND % 4 == 0;
-    template <int G>
-    static constexpr int chunks() { return (MG::template Set<G>::N + 3) / 4; }
-    template <int G = 0>
-    static constexpr int max_chunks() {
-        if constexpr (G + 1 < MG::COUNT) {
-            return chunks<G>() > max_chunks<G + 1>() ? chunks<G>() : max_chunks<G + 1>();
-        } else {
-            return chunks<G>();
-        }
-    }
     // exchange floats per pair, TS / 4 odd (as QuadCfg::TS)
-    static constexpr int TS = (NC + max_chunks()) * 16 + 4;
+    static constexpr int TS = (NC + max_chunks<MG>()) * 16 + 4;
 };
 
 // One tile's sums over its sites for the harmonics of MR (and the radial terms with RAD): dE/dr and
@@ -235,8 +139,8 @@ __device__ __forceinline__ void quad_adjoint_sums(const nepx_pair_model& m, cons
     // ---- B = dE/dA = 2 K^2 dE/dg_ang[n][l] A: this lane's column of chunk d is slot 4d + q ----
     static_for<LC>([&](auto dc) {
         constexpr int d = decltype(dc)::value;
-        constexpr float w0 = MS::two_k2(4 * d), w1 = MS::two_k2(4 * d + 1), w2 = MS::two_k2(4 * d + 2),
-                        w3 = MS::two_k2(4 * d + 3);
+        constexpr float w0 = 2.f * MS::k2(4 * d), w1 = 2.f * MS::k2(4 * d + 1), w2 = 2.f * MS::k2(4 * d + 2),
+                        w3 = 2.f * MS::k2(4 * d + 3);
         constexpr int a0 = MS::row_of(4 * d), a1 = MS::row_of(4 * d + 1), a2 = MS::row_of(4 * d + 2),
                       a3 = MS::row_of(4 * d + 3);
         const float kw = sel4(q, w0, w1, w2, w3);

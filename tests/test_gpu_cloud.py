@@ -70,3 +70,37 @@ def test_cloud_descriptor_rejects_missing_hypers(gpu):
     nep.set_hypers([9, 9, 9, 5.0])
     with pytest.raises(NotImplementedError):
         nep.get_g_fast()
+
+
+@pytest.mark.parametrize("hyp", [(11, 6, 4), (10, 8, 4), (17, 6, 6), (10, 10, 10)])
+@pytest.mark.parametrize("nd,P", [(2, 1), (3, 15), (4, 16), (5, 17), (31, 33), (64, 40), (65, 40), (130, 19), (6, 70001)])
+def test_cloud_descriptor_tile_edges(gpu, hyp, nd, P):
+    """Four lanes per cloud, 16 clouds per tile: site counts off the quad and on both sides of the staging
+    limit (64), ragged last tiles, and more tiles than blocks, weighted, against the FP64 oracle."""
+    from nepx import ops
+    rng = np.random.default_rng(100 * nd + P)
+    X = rng.normal(0, 1.0, (P, nd, 3)).astype(np.float32)
+    w = rng.uniform(0.5, 2.0, nd).astype(np.float32)
+    G = ops.cloud_descriptor(torch.from_numpy(X).to(gpu), *hyp, 6.0, weights=w).cpu().numpy()
+    pick = np.unique(np.concatenate([np.arange(min(P, 40)), np.arange(max(0, P - 40), P)]))
+    G64 = O.descriptor(X[pick].astype(np.float64), 6.0, *hyp, weights=w.astype(np.float64))
+    assert np.all(np.isfinite(G)) and _rowwise(G[pick], G64) < 1e-5
+
+
+def test_cloud_descriptor_into_an_unaligned_row_block(gpu):
+    """Rows are stored 16 bytes at a time only where the output allows it: the same values 4 bytes off."""
+    import nepx  # noqa: F401
+    from nepx import _lib
+    rng = np.random.default_rng(3)
+    P, nd, hyp = 50, 12, (10, 8, 4)
+    X = torch.from_numpy(rng.normal(0, 1.0, (P, nd, 3)).astype(np.float32)).to(gpu)
+    D, out = 47, []
+    for shift in (0, 1):
+        buf = torch.full((P * D + 4,), float("nan"), device=gpu)
+        G = buf[shift:shift + P * D]
+        _lib.check(_lib.lib.nepx_cloud_descriptor(_lib.ptr(X), P, nd, None, *hyp, 6.0, G.data_ptr(),
+                                                  _lib.stream_handle()), "nepx_cloud_descriptor")
+        torch.cuda.synchronize()
+        assert torch.isnan(buf[:shift]).all() and torch.isnan(buf[shift + P * D:]).all()
+        out.append(G.clone())
+    assert torch.equal(out[0], out[1]) and torch.isfinite(out[0]).all()
