@@ -104,3 +104,20 @@ def test_cloud_descriptor_into_an_unaligned_row_block(gpu):
         assert torch.isnan(buf[:shift]).all() and torch.isnan(buf[shift + P * D:]).all()
         out.append(G.clone())
     assert torch.equal(out[0], out[1]) and torch.isfinite(out[0]).all()
+
+
+@pytest.mark.parametrize("n", [0, 1, 2000, 5578, 17334, 40001])
+def test_featurised_rows_equal_the_device_rows(gpu, n):
+    """get_g_fast copies its rows to the host plainly up to 1 MB and through two 8 MB stages beyond
+    (17,331 rows of 121 floats a stage): the same bits as the descriptors on the GPU, in several
+    chunks as well."""
+    from nepx import ops
+    from nepx.NEP import NEP
+    X = np.random.default_rng(n).normal(0, 1.0, (n, 6, 3)).astype(np.float32)
+    nep = NEP(X)
+    nep.set_hypers([10, 10, 10, 6.0])
+    want = ops.cloud_descriptor(torch.from_numpy(X).to(gpu), 10, 10, 10, 6.0).cpu().numpy()
+    for chunk in (1 << 20, 19000):
+        nep.chunk = chunk
+        G = nep.get_g_fast()
+        assert G.dtype == np.float32 and G.shape == (n, 121) and np.array_equal(G, want)
