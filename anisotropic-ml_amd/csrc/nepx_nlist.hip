@@ -21,10 +21,10 @@ constexpr int kScanBlock = 1024;
 constexpr int kSortMax = 2048;  // longest row the in-LDS sort accepts
 constexpr int kSlotsPerBlock = 1024;
 
+// One wrap of t: past L/2 either way, t moves L towards zero.  (The two tests t > L/2 -> t - L,
+// t < -L/2 -> t + L in turn give the same bits: t - L cannot round below -L/2.)
 __device__ __forceinline__ double wrap1(double t, double L) {
-    t = t > 0.5 * L ? t - L : t;
-    t = t < -0.5 * L ? L + t : t;
-    return t;
+    return fabs(t) > 0.5 * L ? __dsub_rn(t, copysign(L, t)) : t;
 }
 
 // Squared minimum-image distance from (xi, yi, zi) to (xj, yj, zj); t = X_j - X_i.
@@ -59,27 +59,23 @@ __device__ __forceinline__ bool live(const nepx_state& st, int i) {
     return s >= 0 && st.sp[s].active;
 }
 
-__global__ void k_set_flag(int32_t* flags, int idx, int v) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) flags[idx] = v;
-}
-
-// Start of a build step: clear the longest-row flag and, when a rebuild is due, the cell counters.
-__global__ void k_build_begin(int32_t* flags, int32_t* cell_count, int32_t* cell_fill, int64_t nct) {
+// Start of a build step: clear the longest-row flag and, when a rebuild is due, the cell counters.  A
+// forced build requests itself and clears a stale overflow (the flags it sets are not read here).
+__global__ void k_build_begin(int32_t* flags, int32_t* cell_count, int32_t* cell_fill, int64_t nct, int force) {
+    const bool build = force || want_build(flags);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         flags[F_MAXROW] = 0;
         flags[F_LONGSYS] = 0;
+        if (force) {
+            flags[F_REBUILD] = 1;
+            flags[F_OVERFLOW] = 0;
+        }
     }
-    if (!want_build(flags)) return;
+    if (!build) return;
     for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < nct; k += (int64_t)gridDim.x * blockDim.x) {
         cell_count[k] = 0;
         cell_fill[k] = 0;
     }
-}
-
-__global__ void k_zero_i32(int32_t* a, int64_t n, const int32_t* flags) {
-    if (flags && !want_build(flags)) return;
-    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
-        a[k] = 0;
 }
 
 __global__ void k_cells_count(nepx_state st, nepx_nlist nl) {
@@ -101,34 +97,70 @@ __global__ void k_cells_count(nepx_state st, nepx_nlist nl) {
     atomicAdd(&nl.cell_count[c], 1);
 }
 
-// Exclusive scan of a[0..n) into out[0..n]; out[n] = total.  One block.
-__device__ void block_exclusive_scan(const int32_t* a, int32_t* out, int n) {
-    __shared__ int32_t buf[kScanBlock];
-    __shared__ int32_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < n; base += kScanBlock) {
-        const int k = base + threadIdx.x;
-        const int32_t v = k < n ? a[k] : 0;
-        buf[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < kScanBlock; off <<= 1) {
-            int32_t add = threadIdx.x >= off ? buf[threadIdx.x - off] : 0;
-            __syncthreads();
-            buf[threadIdx.x] += add;
-            __syncthreads();
+// Exclusive scan of a[0..n) into out (which may be a); returns the total.  One block of kScanBlock
+// threads, kScanPer consecutive entries a thread, the next entries loaded while these are summed.
+constexpr int kScanPer = 8;
+__device__ int block_exclusive_scan(const int32_t* a, int32_t* out, int n) {
+    __shared__ int32_t wsum[kScanBlock / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int32_t v[kScanPer];
+    auto load = [&](int base) {
+        const int k0 = base + threadIdx.x * kScanPer;
+#pragma unroll
+        for (int r = 0; r < kScanPer; ++r) v[r] = k0 + r < n ? a[k0 + r] : 0;
+    };
+    int carry = 0;
+    load(0);
+    for (int base = 0; base < n; base += kScanBlock * kScanPer) {
+        int32_t x[kScanPer], t = 0;
+#pragma unroll
+        for (int r = 0; r < kScanPer; ++r) {
+            x[r] = t;
+            t += v[r];
         }
-        if (k < n) out[k] = carry + buf[threadIdx.x] - v;
+        load(base + kScanBlock * kScanPer);  // past this chunk, so `out` may be `a`
+        int inc = t;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(inc, o, 64);
+            inc += lane >= o ? u : 0;
+        }
+        if (lane == 63) wsum[w] = inc;
         __syncthreads();
-        if (threadIdx.x == kScanBlock - 1) carry += buf[kScanBlock - 1];
-        __syncthreads();
+        int before = carry, all = 0;
+#pragma unroll
+        for (int k = 0; k < kScanBlock / 64; ++k) {
+            const int u = wsum[k];
+            before += k < w ? u : 0;
+            all += u;
+        }
+        before += inc - t;
+        const int k0 = base + threadIdx.x * kScanPer;
+#pragma unroll
+        for (int r = 0; r < kScanPer; ++r)
+            if (k0 + r < n) out[k0 + r] = before + x[r];
+        carry += all;
+        __syncthreads();  // wsum is read before the next chunk's sums
     }
-    if (threadIdx.x == 0) out[n] = carry;
+    return carry;
 }
 
-__global__ __launch_bounds__(kScanBlock) void k_scan_cells(nepx_nlist nl) {
+// Cells are scanned up to the last one a system uses (the counters are also scratch of 2 n entries).
+__global__ __launch_bounds__(kScanBlock) void k_scan_cells(nepx_state st, nepx_nlist nl) {
     if (!want_build(nl.flags)) return;
-    block_exclusive_scan(nl.cell_count, nl.cell_start, nl.n_cells_total);
+    __shared__ int used;
+    if (threadIdx.x == 0) used = 0;
+    __syncthreads();
+    int m = 0;
+    for (int s = threadIdx.x; s < st.n_sys; s += kScanBlock) {
+        const int nc = st.sp[s].nc, e = nc > 0 ? st.sp[s].cell_off + nc * nc * nc : 0;
+        m = e > m ? e : m;
+    }
+    if (m > 0) atomicMax(&used, m);
+    __syncthreads();
+    const int n = used < nl.n_cells_total ? used : nl.n_cells_total;
+    const int total = block_exclusive_scan(nl.cell_count, nl.cell_start, n);
+    if (threadIdx.x == 0) nl.cell_start[n] = total;
 }
 
 __global__ void k_cells_fill(nepx_state st, nepx_nlist nl) {
@@ -144,23 +176,40 @@ __global__ void k_cells_fill(nepx_state st, nepx_nlist nl) {
     reinterpret_cast<double4*>(nl.cell_pos)[pos] = make_double4(st.x[i], st.y[i], st.z[i], 0.0);
 }
 
-// The list build gives each particle a group of kLG lanes.  The lanes walk
-// the candidates j of particle i (27 cells, or the whole system when the
-// box is too small for three cells a side) in rounds of kLG: round r of a
-// cell covers its entries r*kLG + sub.  Every lane of a group sees the same
-// cells and rounds (same i), so ballots inside a round are uniform over the
-// group; f(j, valid, d2) is called for each round slot with the squared
-// minimum-image distance d2, valid = false for slots past the end of a cell
-// and for j == i.  Cell candidates' positions come from
-// the cell-ordered copy (contiguous per cell), the same FP64 values as st.x.
-constexpr int kLG = 16;
+// The list build gives each particle a group of LG lanes.  The lanes walk the candidates j of particle
+// i in rounds of LG: round r of a run of cells covers its entries r*LG + sub.  Every lane of a group sees
+// the same runs and rounds (same i), so ballots inside a round are uniform over the group; f(j, valid, d2)
+// is called for each round slot with the squared minimum-image distance d2, valid = false for slots past
+// the end of a run and for j == i.
+//
+// Cells along z are neighbours in memory, so the cells of one (x, y) column that a particle reaches are one
+// run (two where they wrap): 2 R + 1 cells, R = the cells that cover r_list (1 for cells of a side of
+// r_list or more, 2 for half of that, ...), or the whole system when there are no cells.  Candidates'
+// positions come from the cell-ordered copy (contiguous), the same FP64 values as st.x.
+//
+// LG: with 16 lanes a particle, 4,096 particles are one wave per SIMD and the walk waits for memory, so
+// systems of up to kWideGroups particles take a wave per particle (4,097 tetrahedra, a list of 402,000 pairs:
+// the two walks 254 -> 109 us, with cells of half the list radius as well).
+constexpr int kWideGroups = 8192;
 
-__device__ __forceinline__ uint32_t group_mask(uint64_t ballot) {
-    const int gbase = (threadIdx.x & 63) & ~(kLG - 1);
-    return (uint32_t)((ballot >> gbase) & ((1ull << kLG) - 1ull));
+template <int LG>
+__device__ __forceinline__ uint64_t group_mask(uint64_t ballot) {
+    if constexpr (LG == 64) {
+        return ballot;
+    } else {
+        const int gbase = (threadIdx.x & 63) & ~(LG - 1);
+        return (ballot >> gbase) & ((1ull << LG) - 1ull);
+    }
 }
 
-template <class F>
+// Cells each way that cover r (at least one); nc = floor(L / r) gives 1 whatever the rounding.
+__device__ __forceinline__ int cell_reach(double r, double L, int nc) {
+    const double f = r * (double)nc / L;
+    if (f <= 1.0 + 1e-9) return 1;
+    return f < (double)nc ? (int)ceil(f - 1e-9) : nc;
+}
+
+template <int LG, class F>
 __device__ __forceinline__ void for_candidates(const nepx_state& st, const nepx_nlist& nl, int i, int sub, F&& f) {
     const int s = st.sys[i];
     const nepx_sysparam& sp = st.sp[s];
@@ -168,7 +217,7 @@ __device__ __forceinline__ void for_candidates(const nepx_state& st, const nepx_
     const double xi = st.x[i], yi = st.y[i], zi = st.z[i];
     double tx, ty, tz;
     if (sp.nc <= 0) {
-        for (int base = sp.p_start; base < sp.p_end; base += kLG) {
+        for (int base = sp.p_start; base < sp.p_end; base += LG) {
             const int j = base + sub;
             const bool valid = j < sp.p_end && j != i && st.sys[j] == s;
             const int jj = valid ? j : i;
@@ -178,17 +227,20 @@ __device__ __forceinline__ void for_candidates(const nepx_state& st, const nepx_
         return;
     }
     const double4* cpos = reinterpret_cast<const double4*>(nl.cell_pos);
-    const int nc = sp.nc;
+    const int nc = sp.nc, R = cell_reach(sp.r_list, L, nc);
+    const int span = 2 * R + 1 < nc ? 2 * R + 1 : nc;  // distinct cells a side
     const int cx = cell_coord(st.x[i], L, nc), cy = cell_coord(st.y[i], L, nc), cz = cell_coord(st.z[i], L, nc);
-    for (int dx = -1; dx <= 1; ++dx) {
-        const int ax = (cx + dx + nc) % nc;
-        for (int dy = -1; dy <= 1; ++dy) {
-            const int ay = (cy + dy + nc) % nc;
-            for (int dz = -1; dz <= 1; ++dz) {
-                const int az = (cz + dz + nc) % nc;
-                const int c = sp.cell_off + (ax * nc + ay) * nc + az;
-                const int b = nl.cell_start[c], e = nl.cell_start[c + 1];
-                for (int base = b; base < e; base += kLG) {
+    // the column's cells: [z0, z0 + span), of which those past nc wrap to the front
+    const int z0 = span < nc ? (cz - R + nc) % nc : 0;
+    const int first = z0 + span <= nc ? span : nc - z0;
+    for (int dx = 0; dx < span; ++dx) {
+        const int ax = (cx - R + dx + nc) % nc;
+        for (int dy = 0; dy < span; ++dy) {
+            const int col = sp.cell_off + (ax * nc + (cy - R + dy + nc) % nc) * nc;
+            for (int run = 0; run < (first < span ? 2 : 1); ++run) {
+                const int b = nl.cell_start[run ? col : col + z0];
+                const int e = nl.cell_start[run ? col + span - first : col + z0 + first];
+                for (int base = b; base < e; base += LG) {
                     const int k = base + sub;
                     const bool in = k < e;
                     const int j = in ? nl.cell_list[k] : i;
@@ -208,95 +260,176 @@ __device__ __forceinline__ int group_sum(int v) {
     return v;
 }
 
+// Row lengths.  row_start and rrow_start get each row's offset within its block's rows, row_count[b] and
+// rrow_count[b] the block's totals, which k_scan_rows turns into the blocks' offsets.
+template <int LG>
 __global__ __launch_bounds__(kNB) void k_nbr_count(nepx_state st, nepx_nlist nl) {
     if (!want_build(nl.flags)) return;
-    const int i = (blockIdx.x * kNB + threadIdx.x) / kLG;
-    const int sub = threadIdx.x % kLG;
-    if (i >= st.n) return;  // whole groups exit together
+    constexpr int ROWS = kNB / LG;
+    __shared__ int len[2][ROWS];
+    const int r = threadIdx.x / LG, i = blockIdx.x * ROWS + r;
+    const int sub = threadIdx.x % LG;
     int nf = 0, nr = 0;
-    if (live(st, i)) {
+    if (i < st.n && live(st, i)) {  // uniform per group
         const nepx_sysparam& sp = st.sp[st.sys[i]];
         const double r2 = __dmul_rn(sp.r_list, sp.r_list);
-        for_candidates(st, nl, i, sub, [&](int j, bool valid, double d2) {
+        for_candidates<LG>(st, nl, i, sub, [&](int j, bool valid, double d2) {
             if (valid && d2 < r2) {
                 if (j > i) ++nf;
                 else ++nr;
             }
         });
     }
-    nf = group_sum<kLG>(nf);
-    nr = group_sum<kLG>(nr);
+    nf = group_sum<LG>(nf);
+    nr = group_sum<LG>(nr);
     if (sub == 0) {
-        nl.row_count[i] = nf;
-        nl.rrow_count[i] = nr;
+        len[0][r] = nf;
+        len[1][r] = nr;
         if (nf > kSortMax || nr > kSortMax) {
             atomicMax(&nl.flags[F_MAXROW], nf > nr ? nf : nr);
             nl.flags[F_LONGSYS] = st.sys[i] + 1;  // one system holding such a row (any, if several)
         }
     }
+    __syncthreads();
+    if (threadIdx.x < 2 * ROWS) {
+        const int side = threadIdx.x / ROWS, k = threadIdx.x % ROWS;
+        int o = 0;
+        for (int u = 0; u < k; ++u) o += len[side][u];
+        const int row = blockIdx.x * ROWS + k;
+        int32_t* start = side ? nl.rrow_start : nl.row_start;
+        if (row < st.n) start[row] = o;
+        if (k == ROWS - 1) (side ? nl.rrow_count : nl.row_count)[blockIdx.x] = o + len[side][k];
+    }
 }
 
-__global__ __launch_bounds__(kScanBlock) void k_scan_rows(nepx_nlist nl, int n) {
+// Block 0 scans the forward rows, block 1 the reverse rows: the row counts into row starts (PER_ROW), or the
+// blocks' totals in place.
+template <bool PER_ROW>
+__global__ __launch_bounds__(kScanBlock) void k_scan_rows(nepx_nlist nl, int m, int n) {
     if (!want_build(nl.flags)) return;
     if (blockIdx.x == 0) {
-        block_exclusive_scan(nl.row_count, nl.row_start, n);
-        __syncthreads();
+        const int total = block_exclusive_scan(nl.row_count, PER_ROW ? nl.row_start : nl.row_count, m);
         if (threadIdx.x == 0) {
-            nl.flags[F_PL] = nl.row_start[n];
-            if ((int64_t)nl.row_start[n] > nl.cap || nl.flags[F_MAXROW] > kSortMax) nl.flags[F_OVERFLOW] = 1;
+            nl.row_start[n] = total;
+            nl.flags[F_PL] = total;
+            if ((int64_t)total > nl.cap || nl.flags[F_MAXROW] > kSortMax) nl.flags[F_OVERFLOW] = 1;
         }
     } else {
-        block_exclusive_scan(nl.rrow_count, nl.rrow_start, n);
+        const int total = block_exclusive_scan(nl.rrow_count, PER_ROW ? nl.rrow_start : nl.rrow_count, m);
+        if (threadIdx.x == 0) nl.rrow_start[n] = total;
     }
 }
 
 // Same walk as k_nbr_count; each round's accepted candidates are placed by a
 // ballot prefix within the group (no atomics).  The row order this gives
-// depends on the cell lists; k_sort_rows makes it canonical.
+// depends on the cell lists; the sorts make it canonical.
+template <int LG>
 __global__ __launch_bounds__(kNB) void k_nbr_fill(nepx_state st, nepx_nlist nl) {
-    if (!want_build(nl.flags) || nl.flags[F_OVERFLOW]) return;
-    const int i = (blockIdx.x * kNB + threadIdx.x) / kLG;
-    const int sub = threadIdx.x % kLG;
-    if (i >= st.n || !live(st, i)) return;  // uniform per group
+    if (!want_build(nl.flags)) return;
+    const int i = (blockIdx.x * kNB + threadIdx.x) / LG;
+    const int sub = threadIdx.x % LG;
+    if (i >= st.n) return;  // uniform per group
+    int pf = nl.row_count[blockIdx.x] + nl.row_start[i], pr = nl.rrow_count[blockIdx.x] + nl.rrow_start[i];
+    if (sub == 0) {
+        nl.row_start[i] = pf;
+        nl.rrow_start[i] = pr;
+    }
+    if (nl.flags[F_OVERFLOW] || !live(st, i)) return;
     const nepx_sysparam& sp = st.sp[st.sys[i]];
     const double r2 = __dmul_rn(sp.r_list, sp.r_list);
-    const uint32_t below = (1u << sub) - 1u;
-    int pf = nl.row_start[i], pr = nl.rrow_start[i];
-    for_candidates(st, nl, i, sub, [&](int j, bool valid, double d2) {
+    const uint64_t below = (1ull << sub) - 1ull;
+    for_candidates<LG>(st, nl, i, sub, [&](int j, bool valid, double d2) {
         const bool in = valid && d2 < r2;
         const bool fwd = in && j > i, rev = in && j < i;
-        const uint32_t mf = group_mask(__ballot(fwd)), mr = group_mask(__ballot(rev));
+        const uint64_t mf = group_mask<LG>(__ballot(fwd)), mr = group_mask<LG>(__ballot(rev));
         if (fwd) {
-            const int slot = pf + __popc(mf & below);
+            const int slot = pf + __popcll(mf & below);
             nl.nbr[slot] = j;
             nl.slot_row[slot] = i;
         }
-        if (rev) nl.rnbr[pr + __popc(mr & below)] = j;
-        pf += __popc(mf);
-        pr += __popc(mr);
+        if (rev) nl.rnbr[pr + __popcll(mr & below)] = j;
+        pf += __popcll(mf);
+        pr += __popcll(mr);
     });
 }
 
-// Sort each row ascending: one wave per row (blocks of 64 stride over the
-// rows; grid y selects the forward or the reverse rows), bitonic in LDS.  The
-// grid is capped, so the launch costs little when no rebuild is due.
-constexpr int kSortThreads = 64;
-__global__ __launch_bounds__(kSortThreads) void k_sort_rows(nepx_nlist nl, int n) {
-    if (!want_build(nl.flags) || nl.flags[F_OVERFLOW]) return;
-    const int reverse = blockIdx.y;  // y = 0: forward rows, 1: reverse rows
-    __shared__ int32_t buf[kSortMax];
-    const int32_t* start = reverse ? nl.rrow_start : nl.row_start;
-    int32_t* data = reverse ? nl.rnbr : nl.nbr;
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const int b = start[i], len = start[i + 1] - b;
-        if (len <= 1) continue;  // uniform per block
+// ---- row sorts ----------------------------------------------------------------
+// One wave sorts a row.  Up to 64 * kRegRow entries sit in registers, entry k * 64 + lane in register k of
+// the lane: a bitonic network whose strides below 64 exchange lanes (DPP for 1, 2, 4 and 8) and the others
+// registers, no LDS and no barriers (both sorts and the slots of 402,000 pairs: 152 -> 55 us against a
+// network in LDS).  Longer rows (up to kSortMax) sort in the wave's part of LDS.
+constexpr int kSortThreads = 256, kSortWaves = kSortThreads / 64, kRegRow = 8;
+
+template <int STRIDE>
+__device__ __forceinline__ int lane_xor(int v) {
+    if constexpr (STRIDE == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);   // quad 1,0,3,2
+    else if constexpr (STRIDE == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);  // quad 2,3,0,1
+    else if constexpr (STRIDE == 4)  // 7 - i within eight lanes, then 3 - i within four
+        return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
+    else if constexpr (STRIDE == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);  // rotate 16 by 8
+    else return __shfl_xor(v, STRIDE, 64);
+}
+
+template <int K, int SIZE, int STRIDE>
+__device__ __forceinline__ void bitonic_stage(int32_t (&v)[K], int lane) {
+    if constexpr (STRIDE >= 64) {
+        constexpr int RS = STRIDE / 64;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            if ((k & RS) == 0) {
+                const bool up = (k & (SIZE / 64)) == 0;
+                const int32_t a = v[k], b = v[k | RS], lo = a < b ? a : b, hi = a < b ? b : a;
+                v[k] = up ? lo : hi;
+                v[k | RS] = up ? hi : lo;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const bool up = SIZE < 64 ? (lane & SIZE) == 0 : (k & (SIZE / 64)) == 0;
+            const int32_t o = lane_xor<STRIDE>(v[k]);
+            const bool low = ((lane & STRIDE) == 0) == up;  // this lane keeps the smaller
+            v[k] = low ? (v[k] < o ? v[k] : o) : (v[k] < o ? o : v[k]);
+        }
+    }
+}
+template <int K, int SIZE, int STRIDE>
+__device__ __forceinline__ void bitonic_strides(int32_t (&v)[K], int lane) {
+    bitonic_stage<K, SIZE, STRIDE>(v, lane);
+    if constexpr (STRIDE > 1) bitonic_strides<K, SIZE, STRIDE / 2>(v, lane);
+}
+template <int K, int SIZE = 2>
+__device__ __forceinline__ void bitonic_sort(int32_t (&v)[K], int lane) {
+    bitonic_strides<K, SIZE, SIZE / 2>(v, lane);
+    if constexpr (SIZE < 64 * K) bitonic_sort<K, SIZE * 2>(v, lane);
+}
+
+// load(k) gives entry k of the row, store(k, v) takes the sorted entry k.
+template <int K, class Load, class Store>
+__device__ __forceinline__ void sort_in_registers(int len, int lane, Load&& load, Store&& store) {
+    int32_t v[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = k * 64 + lane < len ? load(k * 64 + lane) : 0x7fffffff;
+    bitonic_sort<K>(v, lane);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if (k * 64 + lane < len) store(k * 64 + lane, v[k]);
+}
+
+template <class Load, class Store>
+__device__ __forceinline__ void sort_row(int len, int lane, int32_t* buf, Load&& load, Store&& store) {
+    if (len <= 64) sort_in_registers<1>(len, lane, load, store);
+    else if (len <= 128) sort_in_registers<2>(len, lane, load, store);
+    else if (len <= 256) sort_in_registers<4>(len, lane, load, store);
+    else if (len <= 64 * kRegRow) sort_in_registers<kRegRow>(len, lane, load, store);
+    else {
         int p2 = 1;
         while (p2 < len) p2 <<= 1;
-        for (int k = threadIdx.x; k < p2; k += kSortThreads) buf[k] = k < len ? data[b + k] : 0x7fffffff;
-        __syncthreads();
+        for (int k = lane; k < p2; k += 64) buf[k] = k < len ? load(k) : 0x7fffffff;
+        wave_lds_order();
         for (int size = 2; size <= p2; size <<= 1) {
             for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                for (int k = threadIdx.x; k < p2; k += kSortThreads) {
+                for (int k = lane; k < p2; k += 64) {
                     const int partner = k ^ stride;
                     if (partner > k) {
                         const bool up = (k & size) == 0;
@@ -307,49 +440,230 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_rows(nepx_nlist nl, int n
                         }
                     }
                 }
-                __syncthreads();
+                wave_lds_order();
             }
         }
-        for (int k = threadIdx.x; k < len; k += kSortThreads) data[b + k] = buf[k];
-        __syncthreads();
+        for (int k = lane; k < len; k += 64) store(k, buf[k]);
+        wave_lds_order();
     }
 }
 
-// Reverse entries hold the partner i; replace it by the slot of (i, k) in row i
-// (binary search in the sorted row).  kLG lanes per particle k.
-__global__ __launch_bounds__(kNB) void k_rev_slots(nepx_nlist nl, int n) {
+// Forward rows ascending in j.  The grid is capped, so the launch costs little when no rebuild is due.
+__global__ __launch_bounds__(kSortThreads) void k_sort_rows(nepx_nlist nl, int n) {
     if (!want_build(nl.flags) || nl.flags[F_OVERFLOW]) return;
-    const int k = (blockIdx.x * kNB + threadIdx.x) / kLG;
-    const int sub = threadIdx.x % kLG;
-    if (k >= n) return;
-    for (int e = nl.rrow_start[k] + sub; e < nl.rrow_start[k + 1]; e += kLG) {
-        const int i = nl.rnbr[e];
-        int lo = nl.row_start[i], hi = nl.row_start[i + 1] - 1, slot = -1;
-        while (lo <= hi) {
-            const int mid = (lo + hi) >> 1;
-            const int v = nl.nbr[mid];
-            if (v == k) {
-                slot = mid;
-                break;
-            }
-            if (v < k) lo = mid + 1;
-            else hi = mid - 1;
-        }
-        if (slot < 0) nl.flags[F_OVERFLOW] = 2;  // inconsistent list: never expected
-        nl.rnbr[e] = slot;
-        if (nl.rpos && slot >= 0) nl.rpos[slot] = e;  // where the reverse row of k holds this slot
+    __shared__ int32_t buf[kSortWaves][kSortMax];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = blockIdx.x * kSortWaves + w; i < n; i += gridDim.x * kSortWaves) {
+        const int b = nl.row_start[i], len = nl.row_start[i + 1] - b;
+        if (len <= 1) continue;  // uniform per wave
+        int32_t* row = nl.nbr + b;
+        sort_row(len, lane, buf[w], [&](int k) { return row[k]; }, [&](int k, int32_t v) { row[k] = v; });
     }
 }
 
-__global__ void k_build_finish(nepx_nlist nl) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && want_build(nl.flags)) {
+// Reverse entries hold the partner i; each becomes the slot of (i, k) in row i (binary search in the sorted
+// row), and the slots are sorted, which orders them by i as the rows are in slot order.  The last block to
+// arrive marks the build done: every block has read the flags by then, and nothing else is handed over.
+__global__ __launch_bounds__(kSortThreads) void k_rev_rows(nepx_nlist nl, int n) {
+    if (!want_build(nl.flags)) return;
+    __shared__ int32_t buf[kSortWaves][kSortMax];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool skip = nl.flags[F_OVERFLOW] != 0;
+    for (int k = blockIdx.x * kSortWaves + w; k < n && !skip; k += gridDim.x * kSortWaves) {
+        const int b = nl.rrow_start[k], len = nl.rrow_start[k + 1] - b;
+        if (len <= 0) continue;  // uniform per wave
+        int32_t* row = nl.rnbr + b;
+        sort_row(
+            len, lane, buf[w],
+            [&](int e) {
+                const int i = row[e];
+                int lo = nl.row_start[i], hi = nl.row_start[i + 1] - 1, slot = -1;
+                while (lo <= hi) {
+                    const int mid = (lo + hi) >> 1;
+                    const int v = nl.nbr[mid];
+                    if (v == k) {
+                        slot = mid;
+                        break;
+                    }
+                    if (v < k) lo = mid + 1;
+                    else hi = mid - 1;
+                }
+                if (slot < 0) nl.flags[F_OVERFLOW] = 2;  // inconsistent list: never expected
+                return slot;
+            },
+            [&](int e, int32_t slot) {
+                row[e] = slot;
+                if (nl.rpos && slot >= 0) nl.rpos[slot] = b + e;  // where the reverse row of k holds this slot
+            });
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(&nl.flags[F_DONE], 1) == (int)gridDim.x - 1) {
+        nl.flags[F_DONE] = 0;
         nl.flags[F_REBUILD] = 0;
         nl.flags[F_SOON] = 0;
         nl.flags[F_BUILDS] += 1;
     }
 }
 
+// ---- whole build of a small list ------------------------------------------------
+// Up to kOneBuild particles in one block and one launch instead of nine: a build point of a captured run
+// costs 5 us instead of 41 when no rebuild is due, which most are not.  A rebuild costs 90 us at 512
+// particles, growing with n^2, against 55 us for the launches above, so the line lies where a rebuild and
+// the two or three build points that follow it cost the same either way.
+// Every distance within a system is taken once (each wave: one particle against 64 later ones, the ballot
+// is a word of its row of the adjacency matrix in LDS; the words before the diagonal are then read off the
+// columns), and rows, reverse rows and slots are read off the matrix in order, so nothing is sorted or
+// searched.
+constexpr int kOneBuild = 640;
+__global__ __launch_bounds__(kScanBlock) void k_build_one(nepx_state st, nepx_nlist nl, int force) {
+    static_assert(kScanBlock >= kOneBuild && kOneBuild % 64 == 0, "one thread per particle");
+    __shared__ uint64_t adj[kOneBuild * (kOneBuild / 64 | 1)];  // rows of an odd number of words: columns on distinct banks
+    __shared__ double pos[3 * kOneBuild];  // then the row starts
+    __shared__ int16_t sysid[kOneBuild];
+    __shared__ int32_t wsum[2][kScanBlock / 64];
+    int32_t* const flags = nl.flags;
+    const bool build = force || want_build(flags);
+    const int stale_overflow = force ? 0 : flags[F_OVERFLOW];
+    if (threadIdx.x == 0) {
+        flags[F_MAXROW] = 0;
+        flags[F_LONGSYS] = 0;
+    }
+    if (!build) return;  // uniform: F_REBUILD and F_SOON are written at the end only
+    const int n = st.n, W = (n + 63) / 64, LD = W | 1, i = threadIdx.x;
+    const int lane = i & 63, wv = __builtin_amdgcn_readfirstlane(i >> 6);
+    if (i < n) {
+        const double x = st.x[i], y = st.y[i], z = st.z[i];
+        st.xb[i] = x;
+        st.yb[i] = y;
+        st.zb[i] = z;
+        pos[i] = x;
+        pos[kOneBuild + i] = y;
+        pos[2 * kOneBuild + i] = z;
+        const int s = st.sys[i];
+        sysid[i] = (int16_t)(s >= 0 && st.sp[s].active ? s : -1);
+    }
+    __syncthreads();
+    for (int r = wv; r < n; r += kScanBlock / 64) {  // uniform per wave
+        const int s = __builtin_amdgcn_readfirstlane((int)sysid[r]);
+        const nepx_sysparam& sp = st.sp[s < 0 ? 0 : s];
+        const double L = sp.L, r2 = __dmul_rn(sp.r_list, sp.r_list);
+        const double xr = pos[r], yr = pos[kOneBuild + r], zr = pos[2 * kOneBuild + r];
+        for (int w = r >> 6; w < W; ++w) {
+            const int j = 64 * w + lane;
+            bool in = false;
+            if (s >= 0 && j < n && j > r && sysid[j] == s) {
+                double tx, ty, tz;
+                in = pos_d2(xr, yr, zr, pos[j], pos[kOneBuild + j], pos[2 * kOneBuild + j], L, tx, ty, tz) < r2;
+            }
+            const uint64_t m = __ballot(in);
+            if (lane == 0) adj[r * LD + w] = m;
+        }
+    }
+    __syncthreads();
+    // partners before r: bit r of their rows (a diagonal word's bits above the diagonal stay as they are)
+    for (int r = wv; r < n; r += kScanBlock / 64) {
+        const int wr = r >> 6;
+        for (int w = 0; w <= wr; ++w) {
+            const int j = 64 * w + lane;
+            const uint64_t m = __ballot(j < r && ((adj[j * LD + wr] >> (r & 63)) & 1ull));
+            if (lane == 0) adj[r * LD + w] = w < wr ? m : adj[r * LD + w] | m;
+        }
+    }
+    __syncthreads();
+    // row lengths (bits above and below the diagonal) and their exclusive scan over the block
+    int len[2] = {0, 0}, inc[2];
+    if (i < n) {
+        for (int w = 0; w < W; ++w) {
+            const uint64_t m = adj[i * LD + w];
+            const uint64_t lo = w < (i >> 6) ? ~0ull : w > (i >> 6) ? 0ull : (1ull << (i & 63)) - 1ull;
+            len[1] += __popcll(m & lo);
+            len[0] += __popcll(m & ~lo);
+        }
+    }
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        inc[side] = len[side];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(inc[side], o, 64);
+            inc[side] += lane >= o ? u : 0;
+        }
+        if (lane == 63) wsum[side][wv] = inc[side];
+    }
+    __syncthreads();
+    int32_t* const rs = reinterpret_cast<int32_t*>(pos);  // the positions are used up
+    int total = 0;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        int before = 0, all = 0;
+        for (int k = 0; k < kScanBlock / 64; ++k) {
+            before += k < wv ? wsum[side][k] : 0;
+            all += wsum[side][k];
+        }
+        const int start = before + inc[side] - len[side];
+        int32_t* const out = side ? nl.rrow_start : nl.row_start;
+        if (i < n) {
+            rs[side * kOneBuild + i] = start;
+            out[i] = start;
+        }
+        if (i == 0) out[n] = all;
+        total = side ? total : all;
+    }
+    const bool over = (int64_t)total > nl.cap;
+    __syncthreads();
+    if (!over && stale_overflow == 0 && i < n) {  // each thread writes its particle's rows
+        int pf = rs[i], pr = rs[kOneBuild + i];
+        for (int w = 0; w < W; ++w) {
+            uint64_t m = adj[i * LD + w];
+            while (m) {
+                const int j = 64 * w + __builtin_ctzll(m);
+                m &= m - 1ull;
+                if (j > i) {
+                    nl.nbr[pf] = j;
+                    nl.slot_row[pf] = i;
+                    ++pf;
+                } else {  // the slot of (j, i) is past row j's partners between j and i
+                    int slot = rs[j];
+                    for (int u = j >> 6; u <= (i >> 6); ++u) {
+                        uint64_t q = adj[j * LD + u];
+                        if (u == (j >> 6)) q &= ~((1ull << (j & 63)) - 1ull);
+                        if (u == (i >> 6)) q &= (1ull << (i & 63)) - 1ull;
+                        slot += __popcll(q);
+                    }
+                    nl.rnbr[pr] = slot;
+                    if (nl.rpos) nl.rpos[slot] = pr;
+                    ++pr;
+                }
+            }
+        }
+    }
+    if (i == 0) {
+        flags[F_PL] = total;
+        flags[F_OVERFLOW] = over ? 1 : stale_overflow;
+        flags[F_REBUILD] = 0;
+        flags[F_SOON] = 0;
+        flags[F_BUILDS] += 1;
+    }
+}
+
 // ---- explicit pair list (API path) ----------------------------------------
+// Requests a "build" so that the shared kernels run, clears the overflow, the row counts and the rows' fill
+// counters (2 n entries of the cell scratch).
+__global__ void k_pairs_begin(nepx_nlist nl, int n) {
+    const int k = blockIdx.x * kNB + threadIdx.x;
+    if (k == 0) {
+        nl.flags[F_REBUILD] = 1;
+        nl.flags[F_OVERFLOW] = 0;
+        nl.flags[F_MAXROW] = 0;
+        nl.flags[F_LONGSYS] = 0;
+    }
+    if (k <= n) {
+        nl.row_count[k] = 0;
+        nl.rrow_count[k] = 0;
+    }
+    if (k < 2 * n) nl.cell_fill[k] = 0;
+}
+
 __global__ void k_pairs_count(nepx_nlist nl, const int64_t* pairs, int64_t m, int n) {
     const int64_t k = blockIdx.x * (int64_t)kNB + threadIdx.x;
     if (k >= m) return;
@@ -657,26 +971,32 @@ extern "C" int nepx_nlist_build(nepx_state* st, nepx_nlist* nl, int32_t force, v
     NEPX_REQUIRE(((uintptr_t)nl->cell_pos & 31) == 0, NEPX_EINVAL, "cell_pos must be 32-byte aligned");
     hipStream_t s = as_stream(stream);
     const int n = st->n;
-    const int gb = blocks_for(n, kNB);
-    if (force) {  // a forced build starts clean: request it and clear a stale overflow
-        hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(64), 0, s, nl->flags, F_REBUILD, 1);
-        hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(64), 0, s, nl->flags, F_OVERFLOW, 0);
+    if (n <= kOneBuild && st->n_sys <= INT16_MAX) {
+        hipLaunchKernelGGL(k_build_one, dim3(1), dim3(kScanBlock), 0, s, *st, *nl, force ? 1 : 0);
         NEPX_LAUNCH_CHECK();
+        return NEPX_OK;
     }
+    const int gb = blocks_for(n, kNB);
     const int nct = nl->n_cells_total > 0 ? nl->n_cells_total : 1;
+    const int gs = blocks_for(n, kSortWaves) < 4096 ? blocks_for(n, kSortWaves) : 4096;
     hipLaunchKernelGGL(k_build_begin, dim3(blocks_for(nct, kNB)), dim3(kNB), 0, s, nl->flags, nl->cell_count,
-                       nl->cell_fill, (int64_t)nct);
+                       nl->cell_fill, (int64_t)nct, force ? 1 : 0);
     hipLaunchKernelGGL(k_cells_count, dim3(gb), dim3(kNB), 0, s, *st, *nl);
-    hipLaunchKernelGGL(k_scan_cells, dim3(1), dim3(kScanBlock), 0, s, *nl);
+    hipLaunchKernelGGL(k_scan_cells, dim3(1), dim3(kScanBlock), 0, s, *st, *nl);
     hipLaunchKernelGGL(k_cells_fill, dim3(gb), dim3(kNB), 0, s, *st, *nl);
-    const int gg = blocks_for((int64_t)n * kLG, kNB);
-    hipLaunchKernelGGL(k_nbr_count, dim3(gg), dim3(kNB), 0, s, *st, *nl);
-    hipLaunchKernelGGL(k_scan_rows, dim3(2), dim3(kScanBlock), 0, s, *nl, n);
-    hipLaunchKernelGGL(k_nbr_fill, dim3(gg), dim3(kNB), 0, s, *st, *nl);
-    const int gs = n < 16384 ? n : 16384;
-    hipLaunchKernelGGL(k_sort_rows, dim3(gs, 2), dim3(kSortThreads), 0, s, *nl, n);
-    hipLaunchKernelGGL(k_rev_slots, dim3(gg), dim3(kNB), 0, s, *nl, n);
-    hipLaunchKernelGGL(k_build_finish, dim3(1), dim3(64), 0, s, *nl);
+#define NEPX_ROWS(LG)                                                                                     \
+    const int gg = blocks_for((int64_t)n * LG, kNB);                                                      \
+    hipLaunchKernelGGL(k_nbr_count<LG>, dim3(gg), dim3(kNB), 0, s, *st, *nl);                             \
+    hipLaunchKernelGGL(k_scan_rows<false>, dim3(2), dim3(kScanBlock), 0, s, *nl, gg, n);                  \
+    hipLaunchKernelGGL(k_nbr_fill<LG>, dim3(gg), dim3(kNB), 0, s, *st, *nl)
+    if (n <= kWideGroups) {
+        NEPX_ROWS(64);
+    } else {
+        NEPX_ROWS(16);
+    }
+#undef NEPX_ROWS
+    hipLaunchKernelGGL(k_sort_rows, dim3(gs), dim3(kSortThreads), 0, s, *nl, n);
+    hipLaunchKernelGGL(k_rev_rows, dim3(gs), dim3(kSortThreads), 0, s, *nl, n);
     NEPX_LAUNCH_CHECK();
     return NEPX_OK;
 }
@@ -689,33 +1009,22 @@ extern "C" int nepx_nlist_from_pairs(nepx_state* st, nepx_nlist* nl, const int64
     NEPX_REQUIRE(m <= nl->cap, NEPX_ECAP, "%lld pairs exceed list capacity %lld", (long long)m,
                  (long long)nl->cap);
     NEPX_REQUIRE(nl->cell_fill && nl->cell_count, NEPX_EINVAL, "null scratch buffer");
+    // per-row fill counters reuse the cell scratch
+    NEPX_REQUIRE(nl->n_cells_total >= 2 * st->n, NEPX_ECAP, "cell scratch (%d) smaller than 2*n (%d)",
+                 nl->n_cells_total, 2 * st->n);
     hipStream_t s = as_stream(stream);
     const int n = st->n;
-    // flags: request a "build" so the shared kernels run, clear overflow
-    hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(64), 0, s, nl->flags, F_REBUILD, 1);
-    hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(64), 0, s, nl->flags, F_OVERFLOW, 0);
-    hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(64), 0, s, nl->flags, F_MAXROW, 0);
-    hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(64), 0, s, nl->flags, F_LONGSYS, 0);
-    hipLaunchKernelGGL(k_zero_i32, dim3(blocks_for(n + 1, kNB)), dim3(kNB), 0, s, nl->row_count,
-                       (int64_t)(n + 1), nullptr);
-    hipLaunchKernelGGL(k_zero_i32, dim3(blocks_for(n + 1, kNB)), dim3(kNB), 0, s, nl->rrow_count,
-                       (int64_t)(n + 1), nullptr);
+    const int gs = blocks_for(n, kSortWaves) < 4096 ? blocks_for(n, kSortWaves) : 4096;
+    hipLaunchKernelGGL(k_pairs_begin, dim3(blocks_for(2 * (int64_t)n + 1, kNB)), dim3(kNB), 0, s, *nl, n);
     if (m > 0)
         hipLaunchKernelGGL(k_pairs_count, dim3(blocks_for(m, kNB)), dim3(kNB), 0, s, *nl, pairs, m, n);
     hipLaunchKernelGGL(k_rows_maxlen, dim3(blocks_for(n, kNB)), dim3(kNB), 0, s, *nl, n);
-    hipLaunchKernelGGL(k_scan_rows, dim3(2), dim3(kScanBlock), 0, s, *nl, n);
-    // per-row fill counters reuse the cell scratch when it is large enough
-    NEPX_REQUIRE(nl->n_cells_total >= 2 * n, NEPX_ECAP, "cell scratch (%d) smaller than 2*n (%d)",
-                 nl->n_cells_total, 2 * n);
-    hipLaunchKernelGGL(k_zero_i32, dim3(blocks_for(2 * n, kNB)), dim3(kNB), 0, s, nl->cell_fill,
-                       (int64_t)(2 * n), nullptr);
+    hipLaunchKernelGGL(k_scan_rows<true>, dim3(2), dim3(kScanBlock), 0, s, *nl, n, n);
     if (m > 0)
         hipLaunchKernelGGL(k_pairs_fill, dim3(blocks_for(m, kNB)), dim3(kNB), 0, s, *nl, pairs, m,
                            nl->cell_fill, nl->cell_fill + n);
-    const int gs = n < 16384 ? n : 16384;
-    hipLaunchKernelGGL(k_sort_rows, dim3(gs, 2), dim3(kSortThreads), 0, s, *nl, n);
-    hipLaunchKernelGGL(k_rev_slots, dim3(blocks_for((int64_t)n * kLG, kNB)), dim3(kNB), 0, s, *nl, n);
-    hipLaunchKernelGGL(k_build_finish, dim3(1), dim3(64), 0, s, *nl);
+    hipLaunchKernelGGL(k_sort_rows, dim3(gs), dim3(kSortThreads), 0, s, *nl, n);
+    hipLaunchKernelGGL(k_rev_rows, dim3(gs), dim3(kSortThreads), 0, s, *nl, n);
     NEPX_LAUNCH_CHECK();
     return NEPX_OK;
 }

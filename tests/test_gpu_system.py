@@ -261,3 +261,91 @@ def test_md_step_c_entry_equals_arena_steps(gpu):
     for k in ("x", "v", "q", "p", "F", "T"):
         assert np.array_equal(x[k], y[k]), k
     assert a.device_steps() == b.device_steps() == 10
+
+
+def _check_list_rows(ar, want):
+    """Rows of the arena's list against `want`, its (i, j) pairs sorted: forward rows, reverse rows (the slots
+    of row k's partners, ascending) and their starts."""
+    lt = {k: ar.lt[k].cpu().numpy() for k in ("nbr", "slot_row", "rnbr", "row_start", "rrow_start", "flags")}
+    M = len(want)
+    assert lt["flags"][2] == M and lt["flags"][0] == 0 and lt["flags"][1] == 0
+    assert np.array_equal(np.stack([lt["slot_row"][:M], lt["nbr"][:M]], 1), want)
+    assert np.array_equal(lt["row_start"], np.searchsorted(want[:, 0], np.arange(ar.n + 1)))
+    order = np.lexsort((want[:, 0], want[:, 1]))
+    assert np.array_equal(lt["rnbr"][:M], order)
+    assert np.array_equal(lt["rrow_start"], np.searchsorted(want[order, 1], np.arange(ar.n + 1)))
+
+
+@pytest.mark.parametrize("shape_name,n,phi", [("cube8", 63, 0.2), ("cube8", 64, 0.2), ("cube8", 65, 0.2),
+                                              ("cube8", 512, 0.3), ("cube8", 640, 0.4), ("cube8", 641, 0.4),
+                                              ("tet10", 900, 0.45), ("tet10", 8192, 0.45), ("tet10", 8193, 0.45),
+                                              ("th_v1", 3000, 0.005), ("cube8", 20000, 0.3)])
+def test_list_build_rows_match_brute_force(gpu, shape_name, n, phi):
+    """Every build path (one block up to 640 particles; a wave per particle up to 8,192; 16 lanes beyond) and
+    both cell sizes, forced and when due after the particles moved, with the optional reverse-row entries."""
+    import nepx
+    from nepx.configs import make_system
+    shape = nepx.get_shape(shape_name)
+    phi = min(phi, n * shape.volume / (2.05 * shape.cutoff) ** 3)
+    spec = make_system(shape_name, n, phi, seed=n, non_overlap=False)
+    hyp = (10, 8, 4) if shape_name == "th_v1" else (11, 6, 4)
+    ar = nepx.Arena([spec], shape, hyp, None, device=gpu, reverse_records=True)
+    r = spec.rc + spec.skin
+
+    def brute(x):
+        from scipy.spatial import cKDTree
+        box = np.where(x < 0, x + spec.L, x) % spec.L
+        cand = cKDTree(box, boxsize=spec.L).query_pairs(r * 1.0001, output_type="ndarray")
+        cand.sort(axis=1)
+        cand = cand[O.pair_d2(x, cand[:, 0], cand[:, 1], spec.L) < r * r]
+        return cand[np.lexsort((cand[:, 1], cand[:, 0]))]
+
+    ar.build_list(True)
+    _check_list_rows(ar, brute(spec.x))
+    rpos, rnbr = ar.lt["rpos"].cpu().numpy(), ar.lt["rnbr"].cpu().numpy()
+    M = int(ar.flags()[2])
+    assert np.array_equal(rnbr[rpos[:M]], np.arange(M))
+    builds = int(ar.flags()[4])
+    ar.build_list(False)                      # not due: nothing happens
+    assert int(ar.flags()[4]) == builds
+    x = spec.x + np.random.default_rng(1).uniform(-0.3, 0.3, spec.x.shape)
+    x = np.where(x > 0.5 * spec.L, x - spec.L, np.where(x < -0.5 * spec.L, x + spec.L, x))
+    ar.set_configuration(x)
+    ar.lt["flags"][0] = 1
+    ar.build_list(False)
+    assert int(ar.flags()[4]) == builds + 1
+    _check_list_rows(ar, brute(x))
+
+
+def test_list_build_of_several_small_systems(gpu):
+    """Two systems in one one-block build: no pair across them, and an inactive one drops out."""
+    import nepx
+    from nepx import _lib
+    from nepx.configs import make_system
+    specs = [make_system("cube8", n, 0.2, seed=n, non_overlap=False) for n in (100, 70)]
+    ar = nepx.Arena(specs, nepx.get_shape("cube8"), (11, 6, 4), None, device=gpu)
+    ar.build_list(True)
+    want = [O.brute_pairs(s.x, s.L, s.rc + s.skin) + a for s, a in zip(specs, ar.starts)]
+    _check_list_rows(ar, np.concatenate(want))
+    rec = ar.t["sp"].cpu().numpy().view(_lib.SYSPARAM_DTYPE).copy()
+    rec["active"][0] = 0
+    ar.t["sp"].copy_(torch.from_numpy(rec.view(np.uint8).copy()))
+    ar.build_list(True)
+    _check_list_rows(ar, want[1])
+
+
+def test_explicit_rows_of_every_length_are_sorted(gpu):
+    """All pairs of 1,500 particles in random order: rows of 0 to 1,499 entries take every sort (one to eight
+    registers a lane, LDS beyond 512 entries), forward and reverse."""
+    import nepx
+    from nepx.configs import make_system
+    n = 1500
+    spec = make_system("cube8", n, 0.2, seed=3, non_overlap=False)
+    ar = nepx.Arena([spec], nepx.get_shape("cube8"), (11, 6, 4), None, device=gpu, list_cap=n * n // 2 + 4096)
+    want = np.stack(np.triu_indices(n, 1), 1)
+    rng = np.random.default_rng(5)
+    p = want[rng.permutation(len(want))]
+    flip = rng.random(len(p)) < 0.5
+    p[flip] = p[flip, ::-1]
+    ar.load_pairs(torch.from_numpy(np.ascontiguousarray(p)))
+    _check_list_rows(ar, want)
