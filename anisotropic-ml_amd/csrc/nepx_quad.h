@@ -64,8 +64,9 @@ __device__ __forceinline__ float sel4(int q, float v0, float v1, float v2, float
     return q == 0 ? v0 : q == 1 ? v1 : q == 2 ? v2 : v3;
 }
 
-// Each block takes BLOCK/4 consecutive pairs per iteration (16 per wave);
+// Each block takes blockDim/4 consecutive pairs per iteration (16 per wave);
 // waves share nothing but the network weights, so the loop has no block barriers.
+// BLOCK threads at most; launches for few pairs use fewer (launch_fused_quad).
 template <class Cfg, class N, int PREC, int ACT>
 __global__ __launch_bounds__(QuadCfg<Cfg>::BLOCK) __attribute__((
     amdgpu_waves_per_eu(QuadCfg<Cfg>::WAVES_PER_SIMD, QuadCfg<Cfg>::WAVES_PER_SIMD))) void k_fused_quad(
@@ -86,6 +87,10 @@ __global__ __launch_bounds__(QuadCfg<Cfg>::BLOCK) __attribute__((
     __shared__ float4 stab[Cfg::ND];
     using R = NetRun<N, 1, PREC>;
     __shared__ __attribute__((aligned(16))) float wl[weight_lds_floats<N, PREC>()];
+    const int P = n_pairs(np_dev, maxp);
+    const int tag = rev_tag(rv);
+    const int per_block = blockDim.x >> 2;
+    if ((int64_t)blockIdx.x * per_block >= P) return;  // no pairs (the grid is sized by the capacity)
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int a = 0; a < Cfg::ND; ++a) {
@@ -98,8 +103,6 @@ __global__ __launch_bounds__(QuadCfg<Cfg>::BLOCK) __attribute__((
     stage_net<N, PREC>(wl, Wg, Whg, W, WH);
     __syncthreads();
 
-    const int P = n_pairs(np_dev, maxp);
-    const int tag = rev_tag(rv);
     const int lane = threadIdx.x & 63, q = lane & 3, wv = threadIdx.x >> 6, slot = lane >> 2;
     float* const xw = xch[wv];
     float* const xp = xw + slot * Q::TS;  // this pair's exchange area
@@ -126,13 +129,13 @@ __global__ __launch_bounds__(QuadCfg<Cfg>::BLOCK) __attribute__((
     // Two waves per SIMD: each iteration loads the next one's pair records (1 % faster at tet10;
     // with one wave per SIMD, cyl12, the registers they hold cost 4 %).
     constexpr bool AHEAD = Q::WAVES_PER_SIMD > 1;
-    const int stride = gridDim.x * (Q::BLOCK / 4);
+    const int stride = gridDim.x * per_block;
     float4 nqi = make_float4(1.f, 0.f, 0.f, 0.f), nqj = nqi, nt = make_float4(1.f, 0.f, 0.f, 0.f);
     if constexpr (AHEAD) {
-        const int idx0 = blockIdx.x * (Q::BLOCK / 4) + (threadIdx.x >> 2);
+        const int idx0 = blockIdx.x * per_block + (threadIdx.x >> 2);
         if (idx0 < P) load_pair(qf, pi, pj, pt, idx0, nqi, nqj, nt);
     }
-    for (int base = blockIdx.x * (Q::BLOCK / 4); base < P; base += stride) {
+    for (int base = blockIdx.x * per_block; base < P; base += stride) {
         const int idx = base + (threadIdx.x >> 2);
         const bool valid = idx < P;
         float4 qi = nqi, qj = nqj, t = nt;  // lanes past the end keep finite stand-in records

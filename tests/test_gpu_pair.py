@@ -265,6 +265,32 @@ def pair_lanes(request):
     tune.set_launch(tune.Tuning(**old))
 
 
+@pytest.mark.parametrize("n_pairs", [0, 1, 63, 64, 65, 20011])
+@pytest.mark.parametrize("shape_name", ["cube8", "tet10"])
+def test_fused_few_pairs_launch_equals_wide_launch(gpu, shape_name, n_pairs):
+    """Up to 65,536 slots of capacity (256 CUs) the four-lane fused kernel runs half blocks; the per-pair
+    results are those of whole blocks bit for bit, and blocks without pairs write nothing (20,011 pairs: two
+    rounds of half blocks)."""
+    import ctypes as C
+    import nepx
+    from nepx import _lib
+    shape, _, T = _inputs(gpu, shape_name, n_pairs=max(n_pairs, 1), seed=21)
+    model = nepx.make_pair_model(shape, (11, 6, 4))
+    net = nepx.EnergyNet.random(40, [64, 64], seed=7, device=gpu)
+    cn = net.cstruct()
+    n_dev = torch.tensor([n_pairs], dtype=torch.int32, device=gpu)
+    res = []
+    for maxp in (65536, 65537):
+        out = torch.full((n_pairs + 1, 12), float("nan"), device=gpu)
+        _lib.check(_lib.lib.nepx_pair_fused(C.byref(model), C.byref(cn), _lib.ptr(T["qf"]), _lib.ptr(T["pi"]),
+                                            _lib.ptr(T["pj"]), _lib.ptr(T["pt"]), _lib.ptr(n_dev), maxp, 100.0,
+                                            _lib.ptr(out), _lib.stream_handle(None)), "nepx_pair_fused")
+        torch.cuda.synchronize()
+        assert torch.isnan(out[n_pairs:]).all() and torch.isfinite(out[:n_pairs]).all()
+        res.append(out[:n_pairs])
+    assert torch.equal(res[0], res[1])
+
+
 @pytest.mark.parametrize("precision", ["f32", "f16x3", "bf16x3", "bf16"])
 @pytest.mark.parametrize("shape_name,hyp,widths", [("tet10", (11, 6, 4), [64, 64]), ("cube8", (11, 6, 4), [64, 64]),
                                                    ("cyl12", (17, 6, 6), [128, 128])])
