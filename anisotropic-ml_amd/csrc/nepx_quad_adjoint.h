@@ -6,12 +6,13 @@
 // and evaluates the sites' geometry, radial functions and harmonics again for every pass, forward and
 // back: eight passes for hypers 10 10 10.  Here the harmonics are cut by m (nepx_msets.h).  Each
 // group of a tile runs on its own wave (hypers 10 10 10: m = {0, 1}, {2, 5}, {3, 4} and {6..10}, 30 of
-// the 120 harmonics each, two waves per SIMD; hypers 10 8 4: all on one wave), and the groups' per-body
-// sums meet in LDS in a fixed order.  The bound is VALU issue (site geometry, radial functions and the
+// the 120 harmonics each, two waves per SIMD; hypers 10 8 4: {0, 1} and {2, 3, 4}), and the groups' per-body
+// sums meet in LDS in a fixed order.  Sites' geometry and radial functions are evaluated once per tile, the
+// trips dealt to the waves, and read from LDS.  The bound is VALU issue (site geometry, radial functions and the
 // per-site gradient sums) and, with two waves per SIMD, the waits of its chains.  8 (12) sites, hypers
-// 10 10 10: 241 pairs 45 -> 13 us (61 -> 15), 20,000 pairs 92 -> 62 us (128 -> 68), 100,001 pairs
-// 310 -> 233 us (419 -> 262); hypers 10 8 4: 241 pairs 15 -> 13 us (20 -> 13), 100,001 pairs 52 -> 40 us
-// (72 -> 50).
+// 10 10 10: 241 pairs 45 -> 13 us (61 -> 13), 20,000 pairs 92 -> 46 us (128 -> 57), 100,001 pairs
+// 310 -> 189 us (419 -> 228); hypers 10 8 4: 241 pairs 15 -> 12 us (20 -> 13), 100,001 pairs 52 -> 47 us
+// (72 -> 59).
 #pragma once
 #include "nepx_msets.h"
 #include "nepx_quad.h"
@@ -59,36 +60,82 @@ __device__ __forceinline__ void angular_site_grad_m(const HarmM<MS>& h, float ux
     gz = Gz;
 }
 
-template <class Cfg>
-struct QuadAdj {
-    using MG = MGroups<Cfg::LMAX>;
-    static constexpr int NA = Cfg::NANG + 1, NC = (NA + 3) / 4, STEPS = Cfg::ND / 4, BLOCK = 64 * MG::COUNT;
-    static constexpr bool OK = Cfg::ND % 4 == 0;
-    // exchange floats per pair, TS / 4 odd (as QuadCfg::TS)
-    static constexpr int TS = (NC + max_chunks<MG>()) * 16 + 4;
+// The adjoint's sets: hypers 10 8 4 take two waves of 12 harmonics each, as one wave's sites would fill the
+// LDS of a whole SIMD's waves.
+template <int LMAX>
+struct AdjSets : MGroups<LMAX> {};
+template <>
+struct AdjSets<4> {
+    static constexpr int COUNT = 2, RAD = 1;
+    static constexpr unsigned MASK[2] = {0x03, 0x1c};
+    template <int G>
+    using Set = MSet<4, MASK[G]>;
 };
 
-// One tile's sums over its sites for the harmonics of MR (and the radial terms with RAD): dE/dr and
+template <class Cfg>
+struct QuadAdj {
+    using MG = AdjSets<Cfg::LMAX>;
+    static constexpr int NA = Cfg::NANG + 1, NC = (NA + 3) / 4, STEPS = Cfg::ND / 4, BLOCK = 64 * MG::COUNT;
+    static constexpr bool OK = Cfg::ND % 4 == 0;
+    // floats per pair of a trip's f and f' and of a wave's harmonics: strides of 4 odd keep the lanes' 64
+    // scalar writes on 64 banks
+    static constexpr int FS = NC * 16 + 4, TS = max_chunks<MG>() * 16 + 4;
+};
+
+// What every wave of a tile needs of its sites, evaluated once: trip s holds the tile's 64 sites 4 s + q.
+template <class Cfg>
+struct QuadSites {
+    using Q = QuadAdj<Cfg>;
+    float4 u[Q::STEPS][64];    // unit vector from the centroid, 1 / distance
+    float4 arm[Q::STEPS][64];  // lever arm about the body's centre, sum_n dE/dg_rad[n] f_n'
+    float f[Q::STEPS][16][Q::FS];   // value 4 ch + i of site 4 s + q at 16 ch + 4 i + q (rows past NANG zero)
+    float df[Q::STEPS][16][Q::FS];  // f_n' of site 4 s + q at 4 NC q + n
+    float s[6][16];                 // the pairs' arm sums s_i and s_j
+};
+
+template <class Cfg>
+__device__ __forceinline__ void quad_adjoint_site(const nepx_pair_model& m, const float4* stab, const PairIn& g,
+                                                  const float* grow, int s, int lane, QuadSites<Cfg>& st) {
+    using Q = QuadAdj<Cfg>;
+    constexpr int NC = Q::NC, NA = Q::NA;
+    const int q = lane & 3, slot = lane >> 2, a = 4 * s + q;
+    const bool bj = a >= Cfg::NS;
+    const float4 b = stab[a];
+    const Mat3 Rb = quat_matrix(bj ? g.qj.x : g.qi.x, bj ? g.qj.y : g.qi.y, bj ? g.qj.z : g.qi.z,
+                                bj ? g.qj.w : g.qi.w);
+    const SiteGeo sg = site_geo_b(Rb, b.x, b.y, b.z, (bj ? g.tx : 0.f) - g.cx, (bj ? g.ty : 0.f) - g.cy,
+                                  (bj ? g.tz : 0.f) - g.cz, 1.f / m.r_nep);
+    float fv[4 * NC], dv[4 * NC];
+#pragma unroll
+    for (int n = NA; n < 4 * NC; ++n) fv[n] = dv[n] = 0.f;
+    float rad = 0.f;
+    radial_derivs<Cfg::NRAD>(sg.rho, [&](int n, float f, float df) {
+        rad += grow[n] * df;
+        if (n < NA) {
+            fv[n] = f;
+            dv[n] = df;
+        }
+    });
+    st.u[s][lane] = make_float4(sg.ux, sg.uy, sg.uz, sg.ir);
+    st.arm[s][lane] = make_float4(sg.ax, sg.ay, sg.az, rad);
+    float* const fp = st.f[s][slot];
+    float* const dp = st.df[s][slot] + 4 * NC * q;
+#pragma unroll
+    for (int n = 0; n < 4 * NC; ++n) fp[16 * (n / 4) + 4 * (n % 4) + q] = fv[n];
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+        *reinterpret_cast<v4f*>(dp + 4 * c) = v4f{dv[4 * c], dv[4 * c + 1], dv[4 * c + 2], dv[4 * c + 3]};
+}
+
+// One tile's sums over its sites for the harmonics of MS (and the radial terms with RAD): dE/dr and
 // arm x dE/dr per body, the same in all four lanes of a pair.
 template <class Cfg, class MS, bool RAD>
-__device__ __forceinline__ void quad_adjoint_sums(const nepx_pair_model& m, const float4* stab, const PairIn& g,
-                                                  const float* grow, float* xp, int q, float (&sum)[12]) {
+__device__ __forceinline__ void quad_adjoint_sums(float inv_rn, const QuadSites<Cfg>& st, const float* grow, float* xp,
+                                                  int lane, float (&sum)[12]) {
     using Q = QuadAdj<Cfg>;
     constexpr int NC = Q::NC, NA = Q::NA, LC = (MS::N + 3) / 4, LMAX = Cfg::LMAX;
     constexpr int GA = Cfg::NRAD + 1;
-    const float inv_rn = 1.f / m.r_nep;
-    auto site = [&](int s, bool& bj) {  // this lane's site a = 4s + q
-        int a = 4 * s + q;
-        bj = a >= Cfg::NS;
-        // opaque: the compiler would keep every trip's geometry and harmonics from the forward for
-        // the adjoint, hundreds of registers
-        asm volatile("" : "+v"(a));
-        const float4 b = stab[a];
-        const Mat3 Rb = quat_matrix(bj ? g.qj.x : g.qi.x, bj ? g.qj.y : g.qi.y, bj ? g.qj.z : g.qi.z,
-                                    bj ? g.qj.w : g.qi.w);
-        return site_geo_b(Rb, b.x, b.y, b.z, (bj ? g.tx : 0.f) - g.cx, (bj ? g.ty : 0.f) - g.cy,
-                          (bj ? g.tz : 0.f) - g.cz, inv_rn);
-    };
+    const int q = lane & 3, slot = lane >> 2;
     // ---- forward: A[n][slot] ----
     v4f Af[NC][LC];
 #pragma unroll
@@ -97,17 +144,10 @@ __device__ __forceinline__ void quad_adjoint_sums(const nepx_pair_model& m, cons
         for (int d = 0; d < LC; ++d) Af[c][d] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int s = 0; s < Q::STEPS; ++s) {
-        bool bj;
-        const SiteGeo sg = site(s, bj);
-        float fv[4 * NC];
-#pragma unroll
-        for (int n = NA; n < 4 * NC; ++n) fv[n] = 0.f;
-        radial_values<Cfg::NANG>(sg.rho, 1.f, [&](int n, float f) { fv[n] = f; });
+        const float4 u = st.u[s][lane];
         HarmM<MS> h;
-        h.eval(sg.ux, sg.uy, sg.uz);
-        wave_lds_order();
-#pragma unroll
-        for (int n = 0; n < 4 * NC; ++n) xp[16 * (n / 4) + 4 * (n % 4) + q] = fv[n];
+        h.eval(u.x, u.y, u.z);
+        wave_lds_order();  // after the previous trip's reads
 #pragma unroll
         for (int mm = 0; mm <= LMAX; ++mm)
 #pragma unroll
@@ -115,26 +155,29 @@ __device__ __forceinline__ void quad_adjoint_sums(const nepx_pair_model& m, cons
 #pragma unroll
                 for (int l = MS::first_l(mm); l <= LMAX; ++l) {
                     const int o = MS::slot(l, mm, part);
-                    xp[16 * (NC + o / 4) + 4 * (o % 4) + q] = h.z(l, mm, part);
+                    xp[16 * (o / 4) + 4 * (o % 4) + q] = h.z(l, mm, part);
                 }
 #pragma unroll
-        for (int o = MS::N; o < 4 * LC; ++o) xp[16 * (NC + o / 4) + 4 * (o % 4) + q] = 0.f;
+        for (int o = MS::N; o < 4 * LC; ++o) xp[16 * (o / 4) + 4 * (o % 4) + q] = 0.f;
         wave_lds_order();
         v4f xf[NC], xz[LC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) xf[c] = *reinterpret_cast<const v4f*>(xp + 16 * c + 4 * q);
+        for (int c = 0; c < NC; ++c) xf[c] = *reinterpret_cast<const v4f*>(st.f[s][slot] + 16 * c + 4 * q);
 #pragma unroll
-        for (int d = 0; d < LC; ++d) xz[d] = *reinterpret_cast<const v4f*>(xp + 16 * (NC + d) + 4 * q);
+        for (int d = 0; d < LC; ++d) xz[d] = *reinterpret_cast<const v4f*>(xp + 16 * d + 4 * q);
+        // each trip's products are one block at the lower wave priority, so that the other waves' VALU
+        // work issues first (as in the fused kernel)
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
                 for (int d = 0; d < LC; ++d)
-                    Af[c][d] = __builtin_amdgcn_mfma_f32_4x4x1f32(
-                        xf[c][k], xz[d][k], Af[c][d], 0, 0, 0);
+                    Af[c][d] = __builtin_amdgcn_mfma_f32_4x4x1f32(xf[c][k], xz[d][k], Af[c][d], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
     }
     // ---- B = dE/dA = 2 K^2 dE/dg_ang[n][l] A: this lane's column of chunk d is slot 4d + q ----
     static_for<LC>([&](auto dc) {
@@ -148,35 +191,21 @@ __device__ __forceinline__ void quad_adjoint_sums(const nepx_pair_model& m, cons
 #pragma unroll
         for (int n = 0; n < NA; ++n) Af[n / 4][d][n % 4] *= kw * row[n * LMAX];
     });
-    float dGr[Cfg::NRAD + 1], ndGr[Cfg::NRAD + 1];
-    float dGr_hi = 0.f;
-    if constexpr (RAD) {
-#pragma unroll
-        for (int n = 0; n <= Cfg::NRAD; ++n) {
-            dGr[n] = grow[n];
-            ndGr[n] = (float)n * dGr[n];
-            if (n >= NA) dGr_hi += dGr[n];
-        }
-    }
     // ---- adjoint ----
     float ig_x = 0.f, ig_y = 0.f, ig_z = 0.f, it_x = 0.f, it_y = 0.f, it_z = 0.f;
     float jg_x = 0.f, jg_y = 0.f, jg_z = 0.f, jt_x = 0.f, jt_y = 0.f, jt_z = 0.f;
 #pragma unroll 1
     for (int s = 0; s < Q::STEPS; ++s) {
-        bool bj;
-        const SiteGeo sg = site(s, bj);
-        float fa[NA], da[NA];
-        float dEdrho = 0.f;
-        if constexpr (RAD) {
-            dEdrho = radial_adjoint<Cfg::NRAD, NA>(sg.rho, dGr, ndGr, dGr_hi, fa, da);
-        } else {
-            radial_derivs<Cfg::NANG>(sg.rho, [&](int n, float f, float df) {
-                fa[n] = f;
-                da[n] = df;
-            });
-        }
+        const float4 u = st.u[s][lane], arm = st.arm[s][lane];
+        float fa[NA];
+        v4f da[NC];
+#pragma unroll
+        for (int n = 0; n < NA; ++n) fa[n] = st.f[s][slot][16 * (n / 4) + 4 * (n % 4) + q];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) da[c] = *reinterpret_cast<const v4f*>(st.df[s][slot] + 4 * NC * q + 4 * c);
         v4f cc[LC], dd[LC];
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int n = 0; n < NA; ++n)
 #pragma unroll
@@ -184,23 +213,29 @@ __device__ __forceinline__ void quad_adjoint_sums(const nepx_pair_model& m, cons
                 const float b = Af[n / 4][d][n % 4];
                 const v4f z4 = {0.f, 0.f, 0.f, 0.f};
                 cc[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(b, fa[n], n == 0 ? z4 : cc[d], 0, 0, 0);
-                dd[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(b, da[n], n == 0 ? z4 : dd[d], 0, 0, 0);
+                dd[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(b, da[n / 4][n % 4], n == 0 ? z4 : dd[d], 0, 0, 0);
             }
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
         HarmM<MS> h;
-        h.eval(sg.ux, sg.uy, sg.uz);
-        float gx, gy, gz;
+        h.eval(u.x, u.y, u.z);
+        float dEdrho = RAD ? arm.w : 0.f, gx, gy, gz;
         angular_site_grad_m<MS>(
-            h, sg.ux, sg.uy,
+            h, u.x, u.y,
             [&](int o, float& c, float& dv) {
                 c = cc[o / 4][o % 4];
                 dv = dd[o / 4][o % 4];
             },
             dEdrho, gx, gy, gz);
+        SiteGeo sg;
+        sg.ux = u.x;
+        sg.uy = u.y;
+        sg.uz = u.z;
+        sg.ir = u.w;
         float ex, ey, ez;
         site_dEdr(sg, dEdrho, inv_rn, gx, gy, gz, ex, ey, ez);
-        const float tx = sg.ay * ez - sg.az * ey, ty = sg.az * ex - sg.ax * ez, tz = sg.ax * ey - sg.ay * ex;
-        const float wj = bj ? 1.f : 0.f, wi = 1.f - wj;
+        const float tx = arm.y * ez - arm.z * ey, ty = arm.z * ex - arm.x * ez, tz = arm.x * ey - arm.y * ex;
+        const float wj = 4 * s + q >= Cfg::NS ? 1.f : 0.f, wi = 1.f - wj;
         ig_x += wi * ex; ig_y += wi * ey; ig_z += wi * ez;
         it_x += wi * tx; it_y += wi * ty; it_z += wi * tz;
         jg_x += wj * ex; jg_y += wj * ey; jg_z += wj * ez;
@@ -220,44 +255,54 @@ __global__ __launch_bounds__((QuadAdj<Cfg>::BLOCK)) __attribute__((amdgpu_waves_
     using Q = QuadAdj<Cfg>;
     using MG = typename Q::MG;
     constexpr int PW = 16, D = Cfg::D, COUNT = MG::COUNT;
+    __shared__ __attribute__((aligned(16))) QuadSites<Cfg> st;
     __shared__ __attribute__((aligned(16))) float xch[COUNT][PW * Q::TS];
     __shared__ float rows[PW * D];
     __shared__ float part[COUNT][12][PW];
     __shared__ float4 stab[Cfg::ND];
+    const int P = n_pairs(np_dev, maxp);
+    if ((int64_t)blockIdx.x * PW >= P) return;  // the grid is sized by the capacity
     if (threadIdx.x < Cfg::ND) {
         const int k = threadIdx.x % Cfg::NS;
         stab[threadIdx.x] = make_float4(m.sites[3 * k], m.sites[3 * k + 1], m.sites[3 * k + 2], 0.f);
     }
-    const int P = n_pairs(np_dev, maxp);
     const int lane = threadIdx.x & 63, q = lane & 3, slot = lane >> 2;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float* const xp = xch[wave] + slot * Q::TS;
+    const float* const grow = rows + slot * D;
+    const float inv_rn = 1.f / m.r_nep;
     for (int base = blockIdx.x * PW; base < P; base += gridDim.x * PW) {  // uniform over the block
         const int idx = base + slot;
         const bool valid = idx < P;
-        float4 qi = make_float4(1.f, 0.f, 0.f, 0.f), qj = qi, t = make_float4(1.f, 0.f, 0.f, 0.f);
-        if (valid) load_pair(qf, pi, pj, pt, idx, qi, qj, t);
         // the tile's dE/dG rows are contiguous
         const int have = (P - base < PW ? P - base : PW) * D;
         for (int k = threadIdx.x; k < PW * D; k += Q::BLOCK) rows[k] = k < have ? dEdG[(size_t)base * D + k] : 0.f;
-        const PairIn g = pair_in<Cfg>(m, qi, qj, t.x, t.y, t.z);
-        __syncthreads();
-        const float* grow = rows + slot * D;
-        float sum[12];
-        if constexpr (COUNT == 1) {
-            quad_adjoint_sums<Cfg, typename MG::template Set<0>, true>(m, stab, g, grow, xp, q, sum);
-        } else {
-            static_for<COUNT>([&](auto gc) {
-                constexpr int G = decltype(gc)::value;
-                if (wave == G)
-                    quad_adjoint_sums<Cfg, typename MG::template Set<G>, G == MG::RAD>(m, stab, g, grow, xp, q, sum);
-            });
-            if (q == 0) {
+        if (wave < Q::STEPS) {  // the trips' sites, dealt to the waves
+            float4 qi = make_float4(1.f, 0.f, 0.f, 0.f), qj = qi, t = make_float4(1.f, 0.f, 0.f, 0.f);
+            if (valid) load_pair(qf, pi, pj, pt, idx, qi, qj, t);
+            const PairIn g = pair_in<Cfg>(m, qi, qj, t.x, t.y, t.z);
+            __syncthreads();  // the rows are there
+            for (int s = wave; s < Q::STEPS; s += COUNT) quad_adjoint_site<Cfg>(m, stab, g, grow, s, lane, st);
+            if (wave == 0 && q == 0) {
+                const float v[6] = {g.six, g.siy, g.siz, g.sjx, g.sjy, g.sjz};
 #pragma unroll
-                for (int c = 0; c < 12; ++c) part[wave][c][slot] = sum[c];
+                for (int c = 0; c < 6; ++c) st.s[c][slot] = v[c];
             }
+        } else {
+            __syncthreads();
         }
-        __syncthreads();  // the groups' sums are there, and every read of the rows is done
+        __syncthreads();  // the sites are there
+        float sum[12];
+        static_for<COUNT>([&](auto gc) {
+            constexpr int G = decltype(gc)::value;
+            if (COUNT == 1 || wave == G)
+                quad_adjoint_sums<Cfg, typename MG::template Set<G>, G == MG::RAD>(inv_rn, st, grow, xp, lane, sum);
+        });
+        if (COUNT > 1 && q == 0) {
+#pragma unroll
+            for (int c = 0; c < 12; ++c) part[wave][c][slot] = sum[c];
+        }
+        __syncthreads();  // the groups' sums are there, and the rows and sites are used up
         if (wave == 0 && q == 0 && valid) {
             if constexpr (COUNT > 1) {
 #pragma unroll
@@ -272,11 +317,12 @@ __global__ __launch_bounds__((QuadAdj<Cfg>::BLOCK)) __attribute__((amdgpu_waves_
             acc.T0x = sum[3]; acc.T0y = sum[4]; acc.T0z = sum[5];
             acc.G1x = sum[6]; acc.G1y = sum[7]; acc.G1z = sum[8];
             acc.T1x = sum[9]; acc.T1y = sum[10]; acc.T1z = sum[11];
-            acc.A0x = g.six; acc.A0y = g.siy; acc.A0z = g.siz;
-            acc.A1x = g.sjx; acc.A1y = g.sjy; acc.A1z = g.sjz;
+            acc.A0x = st.s[0][slot]; acc.A0y = st.s[1][slot]; acc.A0z = st.s[2][slot];
+            acc.A1x = st.s[3][slot]; acc.A1y = st.s[4][slot]; acc.A1z = st.s[5][slot];
             store_out(out, idx, adj_finish<Cfg>(acc), E ? E[idx] : 0.f, clip);
         }
-        // the next tile's sums are written after its first barrier, which wave 0 reaches past these reads
+        // wave 0 reads `part` and `st.s` here; the next tile's are written after a barrier that it reaches past
+        // these reads (st.s by wave 0 itself)
     }
 }
 
