@@ -229,14 +229,26 @@ __global__ __launch_bounds__(kBlock) void k_ffnn(const float* __restrict__ Wg, c
 // barriers, so that L2 latency is covered even with one tile per block.  Every accumulator takes the
 // same products in the same order as ffnn_tiles, and the output sum is formed the same way, so E and
 // dE/dG equal k_ffnn's bit for bit, for any NT.  121 -> 150 x 4: 241 rows 46 -> 18 us, 100,001 rows
-// 1,960 -> 406 us (96 TFLOP/s of padded products, 0.65 of the FP32 rate a large matrix product reaches).
-template <class N, int ACT>
+// 1,960 -> 355 us, 400,003 rows 6,980 -> 1,295 us (120 TFLOP/s of padded products, 0.81 of the FP32 rate a
+// large matrix product reaches).
+//
+// NT: four tiles for ReLU, which keeps one bit per hidden unit for the backward pass; two for deep tanh
+// networks, which keep the activations; one for few pairs.
+//
+// WV waves per block.  With fewer waves than unit blocks (WV = 8 for the ten of a 160-wide layer) each wave
+// takes its block for the NT tiles and one (block, tile) of the EX blocks left over: four tiles make five
+// equal units for each of eight waves, two per SIMD, where ten waves fall 3, 3, 2, 2 on the SIMDs and wait
+// for the fuller ones at every layer's barrier (100,001 rows of 121 -> 150 x 4: 355 against 406 us).  Few
+// tiles take a wave per unit block, the shorter chain, and so do groups of two, which leave four units for
+// eight waves.
+template <class N, int ACT, int WV, int NT_>
 struct SpreadNet {
-    static constexpr int MT = N::MT, NL = N::NL, BLOCK = 64 * MT;
-    // ReLU keeps one bit per hidden unit for the backward pass, tanh the activation itself
-    static constexpr int NT = (ACT == NEPX_ACT_RELU || NL <= 2) ? 4 : 2;
+    static constexpr int MT = N::MT, NL = N::NL, BLOCK = 64 * WV, EX = MT - WV;
+    static_assert(EX >= 0 && N::MD <= WV, "one dE/dG block per wave at most");
+    static constexpr int NT = NT_;
+    static_assert(EX * NT <= WV || EX == 0, "one left-over unit per wave");
     static constexpr int BLOCKS_PER_CU = 2;  // LDS and registers allow two; each hides the other's barriers
-    static constexpr int WAVES_PER_SIMD = (BLOCKS_PER_CU * MT + 3) / 4;
+    static constexpr int WAVES_PER_SIMD = (BLOCKS_PER_CU * WV + 3) / 4;
     // products in order: forward layers 0..NL-1, backward layers NL-1..0; chunks of four k-steps
     static constexpr int chunks(int q) { return (q == 0 ? N::KD : N::KH) / 4; }
     static constexpr int first(int q) { return q == 0 ? 0 : first(q - 1) + chunks(q - 1); }
@@ -248,14 +260,13 @@ struct SpreadNet {
     }
 };
 // Operand chunks in flight per wave: the fewer products a chunk feeds, the further ahead it is read.
-constexpr int spread_depth(int nt) { return nt >= 4 ? 3 : nt == 2 ? 4 : 6; }
+constexpr int spread_depth(int nt) { return nt >= 3 ? 2 : nt == 2 ? 4 : 6; }
 
-template <class N, int ACT, int NT>
+template <class S, class N, int ACT, int WV, int NT>
 __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float en_min, float scale, int D,
                                             const float* __restrict__ G, int P, int tile0, float* __restrict__ E,
                                             float* __restrict__ dEdG,
-                                            v4f (&xs)[2][SpreadNet<N, ACT>::NT][N::MT][64]) {
-    using S = SpreadNet<N, ACT>;
+                                            v4f (&xs)[2][S::NT][N::MT][64]) {
     constexpr NetLayout Lay = N::layout();
     constexpr int MT = N::MT, NL = N::NL, kDepth = spread_depth(NT);
     uint32_t lane = threadIdx.x;
@@ -263,9 +274,12 @@ __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float e
     lane &= 63u;                    // known range: the reads take a scalar base and this offset
     const int g = lane >> 4, pl = lane & 15;
     const int m = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // this wave's 16-unit block
+    // and its left-over unit: block m2 of tile t2 (with fewer than WV of them, some are computed twice)
+    constexpr bool LEFT = S::EX > 0;
+    const int t2 = m % NT, m2 = LEFT ? WV + (m / NT) % S::EX : 0;
     // operands of chunk f of the whole sequence for this wave's block (dE/dG has MD blocks only: the
     // other waves read block 0's there and drop out before using them)
-    float ring[kDepth][4];
+    float ring[kDepth][4], ring2[LEFT ? kDepth : 1][4];
     auto load_chunk = [&](auto fc) {
         constexpr int f = decltype(fc)::value;
         if constexpr (f < S::TOTAL) {
@@ -273,17 +287,23 @@ __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float e
             constexpr int k = q < NL ? q : 2 * NL - 1 - q;
             constexpr int ks = q == 0 ? N::KD : N::KH;
             constexpr int off = (q < NL ? Lay.fwd_off(k) : Lay.bwd_off(k)) + 4 * c * 64;
-            const int mm = (q == 2 * NL - 1 && N::MD < MT && m >= N::MD) ? 0 : m;
+            const int mm = (q == 2 * NL - 1 && N::MD < WV && m >= N::MD) ? 0 : m;
             const float* src = W + (off + mm * ks * 64);
 #pragma unroll
             for (int r = 0; r < 4; ++r) ring[f % kDepth][r] = src[r * 64 + lane];
+            if constexpr (LEFT && q != 2 * NL - 1) {
+                const float* src2 = W + (off + m2 * ks * 64);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ring2[f % kDepth][r] = src2[r * 64 + lane];
+            }
         }
     };
-    auto load4 = [&](const float* src) {  // units 16 m + 4 g + 0..3 of a bias or the output layer
-        const float4 v = *reinterpret_cast<const float4*>(src + 16 * m + 4 * g);
+    auto load4 = [&](const float* src, int mb) {  // units 16 mb + 4 g + 0..3 of a bias or the output layer
+        const float4 v = *reinterpret_cast<const float4*>(src + 16 * mb + 4 * g);
         return v4f{v.x, v.y, v.z, v.w};
     };
-    v4f bias = load4(W + Lay.bias_off(0));  // one layer ahead
+    v4f bias = load4(W + Lay.bias_off(0), m), bias2 = bias;  // one layer ahead
+    if constexpr (LEFT) bias2 = load4(W + Lay.bias_off(0), m2);
     static_for<kDepth>([&](auto f) { load_chunk(f); });
     // the input rows in the B operand's layout: wave c loads chunk c
     if (m < N::MD) {
@@ -301,8 +321,9 @@ __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float e
     }
     __syncthreads();
     // acc += the product q of this wave's block with the vectors in xs[buf]
-    auto product = [&](auto qc, v4f (&acc)[NT]) {
+    auto product = [&](auto qc, v4f (&acc)[NT], v4f& acc2) {
         constexpr int q = decltype(qc)::value, buf = (q < NL ? q : q + 1) & 1;
+        constexpr bool two = LEFT && q != 2 * NL - 1;
         v4f x[2][NT];  // one chunk ahead
 #pragma unroll
         for (int t = 0; t < NT; ++t) x[0][t] = xs[buf][t][0][lane];
@@ -312,50 +333,65 @@ __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float e
 #pragma unroll
                 for (int t = 0; t < NT; ++t) x[(c + 1) & 1][t] = xs[buf][t][c + 1][lane];
             }
+            v4f x2;  // the left-over unit's products come last in the chunk, after this read
+            if constexpr (two) x2 = xs[buf][t2][c][lane];
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ring[f % kDepth][r], x[c & 1][t][r], acc[t], 0, 0, 0);
+            if constexpr (two) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(ring2[f % kDepth][r], x2[r], acc2, 0, 0, 0);
+            }
             load_chunk(std::integral_constant<int, f + kDepth>{});
-            __builtin_amdgcn_sched_barrier(0);  // reads stay this far ahead; all at once they would spill
+            // reads stay this far ahead (all at once they would spill; with a left-over unit the compiler
+            // keeps them apart by itself and the barrier is what spills)
+            if constexpr (!LEFT) __builtin_amdgcn_sched_barrier(0);
         });
     };
     constexpr bool BITS = ACT == NEPX_ACT_RELU;
-    v4f h[BITS ? 1 : NL][BITS ? 1 : NT];  // this wave's activations (tanh)
-    uint32_t on[BITS ? NL : 1] = {};      // its active units (ReLU), bit 4 t + r
+    v4f h[BITS ? 1 : NL][BITS ? 1 : NT + 1];  // this wave's activations (tanh), the left-over unit's at NT
+    uint32_t on[BITS ? NL : 1] = {};          // its active units (ReLU), bit 4 t + r
     auto der = [&](int k, int t, int r) {
         if constexpr (BITS) return (on[k] >> (4 * t + r)) & 1u ? 1.f : 0.f;
         else return act_der(h[k][t][r], ACT);
     };
     static_for<NL>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
-        v4f acc[NT];
+        v4f acc[NT], acc2 = bias2;
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = bias;
-        bias = load4(W + (k + 1 < NL ? Lay.bias_off(k + 1) : Lay.wout_off()));
-        product(kc, acc);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
+        constexpr int next = k + 1 < NL ? Lay.bias_off(k + 1) : Lay.wout_off();
+        bias = load4(W + next, m);
+        if constexpr (LEFT) bias2 = load4(W + next, m2);
+        product(kc, acc, acc2);
+        auto finish = [&](int t, const v4f& a) {
             v4f o;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                o[r] = act_fwd(acc[t][r], ACT);
+                o[r] = act_fwd(a[r], ACT);
                 if constexpr (BITS) on[k] |= (o[r] > 0.f ? 1u : 0u) << (4 * t + r);
             }
             if constexpr (!BITS) h[k][t] = o;
-            xs[(k + 1) & 1][t][m][lane] = o;
-        }
+            return o;
+        };
+#pragma unroll
+        for (int t = 0; t < NT; ++t) xs[(k + 1) & 1][t][m][lane] = finish(t, acc[t]);
+        if constexpr (LEFT) xs[(k + 1) & 1][t2][m2][lane] = finish(NT, acc2);
         __syncthreads();
     });
     // the last layer's deltas (`bias` holds the output layer's weights of this wave's units)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
+    auto last_delta = [&](int t, const v4f& w) {
         v4f d;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) d[r] = scale * bias[r] * der(NL - 1, t, r);
-        xs[(NL + 1) & 1][t][m][lane] = d;
-    }
+        for (int r = 0; r < 4; ++r) d[r] = scale * w[r] * der(NL - 1, t, r);
+        return d;
+    };
+#pragma unroll
+    for (int t = 0; t < NT; ++t) xs[(NL + 1) & 1][t][m][lane] = last_delta(t, bias);
+    if constexpr (LEFT) xs[(NL + 1) & 1][t2][m2][lane] = last_delta(NT, bias2);
     // output layer: wave t forms tile t's sum from the whole last layer, in ffnn_tiles' order
     if (m < NT) {
         const float* wo = W + Lay.wout_off();
@@ -377,24 +413,26 @@ __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float e
     __syncthreads();
     static_for<NL - 1>([&](auto jc) {  // the deltas of layer k - 1 from those of layer k
         constexpr int q = NL + decltype(jc)::value, k = 2 * NL - 1 - q;
-        v4f acc[NT];
+        v4f acc[NT], acc2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-        product(std::integral_constant<int, q>{}, acc);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
+        product(std::integral_constant<int, q>{}, acc, acc2);
+        auto delta = [&](int t, const v4f& a) {
             v4f d;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) d[r] = acc[t][r] * der(k - 1, t, r);
-            xs[q & 1][t][m][lane] = d;
-        }
+            for (int r = 0; r < 4; ++r) d[r] = a[r] * der(k - 1, t, r);
+            return d;
+        };
+#pragma unroll
+        for (int t = 0; t < NT; ++t) xs[q & 1][t][m][lane] = delta(t, acc[t]);
+        if constexpr (LEFT) xs[q & 1][t2][m2][lane] = delta(NT, acc2);
         __syncthreads();
     });
     if (m < N::MD) {  // dE/dG (uniform per wave)
-        v4f acc[NT];
+        v4f acc[NT], none;
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-        product(std::integral_constant<int, 2 * NL - 1>{}, acc);
+        product(std::integral_constant<int, 2 * NL - 1>{}, acc, none);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const int p = (tile0 + t) * 16 + pl;
@@ -407,14 +445,14 @@ __device__ __forceinline__ void ffnn_spread(const float* __restrict__ W, float e
     }
 }
 
-// Each block takes an equal run of tiles, in groups of NT, then of two and one: with many pairs the
+// Each block takes an equal run of tiles, in groups of NT and one of what is left: with many pairs the
 // operand reads are shared four ways and the blocks end together, with few every block has one tile.
-template <class N, int ACT>
-__global__ __launch_bounds__((SpreadNet<N, ACT>::BLOCK)) __attribute__((
-    amdgpu_waves_per_eu(SpreadNet<N, ACT>::WAVES_PER_SIMD, SpreadNet<N, ACT>::WAVES_PER_SIMD))) void k_ffnn_spread(
+template <class N, int ACT, int WV, int NT>
+__global__ __launch_bounds__((SpreadNet<N, ACT, WV, NT>::BLOCK)) __attribute__((
+    amdgpu_waves_per_eu(SpreadNet<N, ACT, WV, NT>::WAVES_PER_SIMD, SpreadNet<N, ACT, WV, NT>::WAVES_PER_SIMD))) void k_ffnn_spread(
     const float* __restrict__ W, float en_min, float scale, int D, const float* __restrict__ G,
     const int32_t* __restrict__ np_dev, int64_t maxp, float* __restrict__ E, float* __restrict__ dEdG) {
-    using S = SpreadNet<N, ACT>;
+    using S = SpreadNet<N, ACT, WV, NT>;
     __shared__ v4f xs[2][S::NT][N::MT][64];  // one layer's outputs: block c of lane l of tile t at [t][c][l]
     const int P = n_pairs(np_dev, maxp);
     const int nt = (P + 15) / 16;
@@ -423,16 +461,18 @@ __global__ __launch_bounds__((SpreadNet<N, ACT>::BLOCK)) __attribute__((
     const int end = tile + per < nt ? tile + per : nt;
     while (tile < end) {  // uniform over the block
         const int left = end - tile;
-        if (S::NT >= 4 && left >= 4) {
-            ffnn_spread<N, ACT, S::NT>(W, en_min, scale, D, G, P, tile, E, dEdG, xs);
-            tile += 4;
-        } else if (left >= 2) {
-            ffnn_spread<N, ACT, 2>(W, en_min, scale, D, G, P, tile, E, dEdG, xs);
-            tile += 2;
-        } else {
-            ffnn_spread<N, ACT, 1>(W, en_min, scale, D, G, P, tile, E, dEdG, xs);
-            tile += 1;
+        auto group = [&](auto nt) {
+            ffnn_spread<S, N, ACT, WV, decltype(nt)::value>(W, en_min, scale, D, G, P, tile, E, dEdG, xs);
+            tile += decltype(nt)::value;
+        };
+        if constexpr (NT >= 4) {
+            if (left >= 4) group(std::integral_constant<int, 4>{});
+            else if (left == 3) group(std::integral_constant<int, 3>{});
         }
+        if constexpr (NT >= 2) {
+            if (left == 2 || (NT < 4 && left > 2)) group(std::integral_constant<int, 2>{});
+        }
+        if (left == 1 || NT == 1) group(std::integral_constant<int, 1>{});
         __syncthreads();  // the last reads of xs are done before the next tiles write it
     }
 }
@@ -917,22 +957,27 @@ static int launch_ffnn(const nepx_net* net, int grid, float scale, int d, const 
 
 // The FP32 network runs on k_ffnn_spread where a block's copy of its operands does not fit in LDS (one
 // wave per tile would read them from L2 for every tile: 60 -> 128 x 2 at 20,000 rows 93 us against
-// 28, 121 -> 150 x 4 536 against 97), and, for the network that fits, up to four tiles per CU (too few
+// 26, 121 -> 150 x 4 536 against 86), and, for the network that fits, up to four tiles per CU (too few
 // for a wave each; beyond, k_ffnn's copy in LDS is as fast); same results.
 template <class T>
 static bool launch_ffnn_spread(const nepx_net* net, float scale, int d, const float* G, const int32_t* np_dev,
                                int64_t maxp, float* E, float* dEdG, void* stream) {
     const int64_t tiles = (maxp + 15) / 16, cus = device_cus();
     if (net->precision != NEPX_NET_F32 || (weights_in_lds<T, NEPX_NET_F32>() && tiles > 4 * cus)) return false;
-#define NEPX_LAUNCH_SPREAD(A)                                                                                   \
-    hipLaunchKernelGGL((k_ffnn_spread<T, A>),                                                                   \
-                       dim3((unsigned)(tiles < SpreadNet<T, A>::BLOCKS_PER_CU * cus                             \
-                                           ? tiles                                                              \
-                                           : SpreadNet<T, A>::BLOCKS_PER_CU * cus)),                            \
-                       dim3(SpreadNet<T, A>::BLOCK), 0, as_stream(stream), net->w_packed, net->en_min, scale, d, G, \
-                       np_dev, maxp, E, dEdG)
-    if (net->act == NEPX_ACT_TANH) NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH);
-    else NEPX_LAUNCH_SPREAD(NEPX_ACT_RELU);
+    constexpr int TANH_NT = T::NL <= 2 ? 4 : 2, TANH_WV = TANH_NT == 4 && T::MT > 8 ? 8 : T::MT;
+    constexpr int RELU_WV = T::MT > 8 ? 8 : T::MT;
+#define NEPX_LAUNCH_SPREAD(A, WV, NT)                                                                              \
+    hipLaunchKernelGGL((k_ffnn_spread<T, A, WV, NT>), dim3((unsigned)(tiles < 2 * cus ? tiles : 2 * cus)),         \
+                       dim3((SpreadNet<T, A, WV, NT>::BLOCK)), 0, as_stream(stream), net->w_packed, net->en_min,   \
+                       scale, d, G, np_dev, maxp, E, dEdG)
+    const bool few = tiles <= 2 * cus;  // one tile per block at most
+    if (net->act == NEPX_ACT_TANH) {
+        if (few) NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH, T::MT, 1);
+        else NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH, TANH_WV, TANH_NT);
+    } else {
+        if (few) NEPX_LAUNCH_SPREAD(NEPX_ACT_RELU, T::MT, 1);
+        else NEPX_LAUNCH_SPREAD(NEPX_ACT_RELU, RELU_WV, 4);
+    }
 #undef NEPX_LAUNCH_SPREAD
     return true;
 }

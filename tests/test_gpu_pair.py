@@ -130,14 +130,14 @@ def test_ffnn_few_pairs_kernel_equals_wide_kernel(gpu, d_in, widths, act):
 @pytest.mark.parametrize("d_in,widths,act", [(121, [150] * 4, "relu"), (121, [150] * 4, "tanh"),
                                              (47, [150] * 4, "relu"), (60, [128, 128], "tanh")])
 def test_ffnn_tile_groups_equal_single_tiles(gpu, d_in, widths, act):
-    """The FP32 network's blocks take equal runs of 16-pair tiles in groups of four, two and one (512
-    blocks on 256 CUs: 3, 5 and 7 tiles per block here, the last row short of a tile); every row equals,
+    """The FP32 network's blocks take equal runs of 16-pair tiles in groups of four to one (512 blocks on
+    256 CUs: 2, 3, 5, 6 and 7 tiles per block here, the last row short of a tile); every row equals,
     bit for bit, the same row of a call small enough for one tile per block."""
     import nepx
     from nepx import ops
     net = nepx.EnergyNet.random(d_in, widths, seed=5, act=act, en_min=-2.0, en_max=3.0, device=gpu, precision="f32")
     g = torch.Generator(device=gpu).manual_seed(4)
-    for per_block in (3, 5, 7):
+    for per_block in (2, 3, 5, 6, 7):
         P = 16 * 512 * per_block - 5
         G = 20.0 * torch.rand((P, d_in), generator=g, device=gpu)
         E, dG = ops.ffnn_forward_backward(net, G)
