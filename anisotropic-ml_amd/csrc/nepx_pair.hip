@@ -91,6 +91,8 @@ __global__ __launch_bounds__(kBlock) NEPX_ADJ_ATTR void k_adjoint(nepx_pair_mode
 // each pass's descriptor entries as k_desc_fwd does; the adjoint leaves each pass's per-body sums
 // in LDS and sums them in pass order, so both give k_desc_fwd's and k_adjoint's results bit for
 // bit (every pass's sums start from zero, as k_adjoint's running sums do not become -0).
+// The forward can also be launched with one pass a block (blockIdx.y, high l first; 64 threads): the
+// time of few pairs is the longest wave's, here one pass instead of two.
 template <class Cfg>
 constexpr int pass_waves() {
     constexpr int np = n_passes(Cfg::NANG, Cfg::LMAX);
@@ -108,6 +110,8 @@ __global__ __launch_bounds__(64 * pass_waves<Cfg>()) NEPX_ADJ_ATTR void k_desc_f
     const float4* __restrict__ pt, const int32_t* __restrict__ np_dev, int64_t maxp, float* __restrict__ G) {
     const int P = n_pairs(np_dev, maxp);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool alone = gridDim.y > 1;  // one pass a block
+    const int pass = (int)gridDim.y - 1 - (int)blockIdx.y;
     for (int idx = blockIdx.x * 64 + (threadIdx.x & 63); idx < P; idx += gridDim.x * 64) {
         float4 qi, qj, t;
         load_pair(qf, pi, pj, pt, idx, qi, qj, t);
@@ -116,7 +120,9 @@ __global__ __launch_bounds__(64 * pass_waves<Cfg>()) NEPX_ADJ_ATTR void k_desc_f
         float* row = G + (size_t)idx * Cfg::D;
         int k = 0;
         for_passes<Cfg>([&](auto range, auto first) {
-            if (pass_owner<Cfg>(k++) == wave) {
+            const bool mine = alone ? k == pass : pass_owner<Cfg>(k) == wave;
+            ++k;
+            if (mine) {
                 using LR = decltype(range);
                 float grad[Cfg::NRAD + 1];
                 float A[Cfg::NANG + 1][LR::N];
@@ -674,13 +680,26 @@ static bool by_passes(int64_t maxp) {
     return !Cfg::ONE_PASS && (maxp + 63) / 64 <= 2 * (int64_t)device_cus();
 }
 static int pass_grid(int64_t maxp) { return (int)((maxp + 63) / 64); }
+// The forward's passes go one to a block while every one of those waves has a SIMD to itself (4 a CU);
+// up to four passes have a wave each already.  hypers 10 10 10, one call, two passes a wave -> one:
+//   4 sites: 241 pairs 16.2 -> 13.0 us, 3,000 16.5 -> 13.6, 8,000 17.4 -> 15.7
+//   6 sites: 241 pairs 21.5 -> 14.9 us, 3,000 22.1 -> 17.0, 8,000 22.9 -> 19.1
+// With more waves than SIMDs it mostly loses: 4 sites, 20,000 pairs 33.7 -> 36.3 us, 100,001 pairs (there
+// against one lane per pair) 110 -> 135 us; 6 sites, 20,000 pairs 44.8 -> 42.6 us, 100,001 pairs 143 -> 166 us.
+template <class Cfg>
+static bool passes_alone(int64_t maxp) {
+    constexpr int np = n_passes(Cfg::NANG, Cfg::LMAX);
+    return np > pass_waves<Cfg>() && (int64_t)pass_grid(maxp) * np <= 4 * (int64_t)device_cus();
+}
 
 template <class T>
 static void launch_desc_fwd(const nepx_pair_model& m, const float* qf, const int32_t* pair_i, const int32_t* pair_j,
                             const float* pair_t, const int32_t* np_dev, int64_t maxp, float* G, void* stream) {
     if constexpr (!T::ONE_PASS) {
         if (by_passes<T>(maxp)) {
-            hipLaunchKernelGGL(k_desc_fwd_passes<T>, dim3(pass_grid(maxp)), dim3(64 * pass_waves<T>()), 0,
+            const bool alone = passes_alone<T>(maxp);
+            const dim3 grid(pass_grid(maxp), alone ? n_passes(T::NANG, T::LMAX) : 1);
+            hipLaunchKernelGGL(k_desc_fwd_passes<T>, grid, dim3(alone ? 64 : 64 * pass_waves<T>()), 0,
                                as_stream(stream), m, (const float4*)qf, pair_i, pair_j, (const float4*)pair_t,
                                np_dev, maxp, G);
             return;

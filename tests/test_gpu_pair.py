@@ -255,6 +255,30 @@ def test_pass_kernels_equal_pair_kernels(gpu, shape_name, hyp):
     assert np.array_equal(o0, o1)
 
 
+@pytest.mark.parametrize("n_pairs", [1, 63, 64, 65, 400])
+@pytest.mark.parametrize("shape_name,hyp", CASES)
+def test_descriptor_launches_equal(gpu, shape_name, hyp, n_pairs):
+    """The capacity picks one pass a block, two passes a wave or one lane per pair (multi-pass
+    shapes); every launch writes the same bits and nothing past the last pair."""
+    import ctypes as C
+    import nepx
+    from nepx import _lib
+    shape, (q, i, j, t), T = _inputs(gpu, shape_name, n_pairs=400, seed=6)
+    model = nepx.make_pair_model(shape, hyp)
+    n_dev = torch.tensor([min(n_pairs, len(i))], dtype=torch.int32, device=gpu)
+    res = []
+    for maxp in (400, 20000, 100000):
+        G = torch.full((401, nepx.n_descriptor(*hyp)), float("nan"), device=gpu)
+        _lib.check(_lib.lib.nepx_descriptor_fwd(C.byref(model), _lib.ptr(T["qf"]), _lib.ptr(T["pi"]),
+                                                _lib.ptr(T["pj"]), _lib.ptr(T["pt"]), _lib.ptr(n_dev), maxp,
+                                                _lib.ptr(G), _lib.stream_handle(None)), "nepx_descriptor_fwd")
+        torch.cuda.synchronize()
+        P = int(n_dev.item())
+        assert torch.isfinite(G[:P]).all() and torch.isnan(G[P:]).all()
+        res.append(G[:P])
+    assert torch.equal(res[0], res[1]) and torch.equal(res[0], res[2])
+
+
 @pytest.fixture(params=[4, 1], ids=["lanes4", "lanes1"])
 def pair_lanes(request):
     """Fused kernel variant: four lanes per pair (site sums on MFMA) or one lane per pair."""
