@@ -128,7 +128,8 @@ typedef struct nepx_nlist {
                                         at the next build point, [8] 1 + a system with a row over 2048
                                         (0: none), [9] filter pass count (the tag of this step's
                                         reverse-order records), [10] tag of the last pass whose pair
-                                        kernel wrote them; others zero */
+                                        kernel wrote them, [11] blocks of the
+                                        build that are done (zero between builds); others zero */
     int32_t* pair_i;                 /* cap: compacted pairs                       */
     int32_t* pair_j;
     float* pair_t;                   /* cap*4: minimum-image t = X_j - X_i (f32)  */
