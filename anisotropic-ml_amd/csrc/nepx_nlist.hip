@@ -41,11 +41,13 @@ __device__ __forceinline__ double pair_d2(const nepx_state& st, double L, int i,
     return pos_d2(st.x[i], st.y[i], st.z[i], st.x[j], st.y[j], st.z[j], L, tx, ty, tz);
 }
 
-// Cell of coordinate x along one side, clamped to [0, nc): NaN and infinities (a faulted
-// system's particles, between the step that went non-finite and its removal) land in the
-// edge cells; the comparisons run in floating point so no out-of-range value is converted.
+// Cell of coordinate x along one side: x is wrapped once, as the pair predicate wraps differences, so a
+// configuration off the box (positions in [0, L), or moved and not folded back) has the cells of its image
+// in the box.  Clamped to [0, nc): NaN and infinities (a faulted system's particles, between the step that
+// went non-finite and its removal) land in the edge cells; the comparisons run in floating point so no
+// out-of-range value is converted.
 __device__ __forceinline__ int cell_coord(double x, double L, int nc) {
-    const double f = floor((x + 0.5 * L) / L * (double)nc);
+    const double f = floor((wrap1(x, L) + 0.5 * L) / L * (double)nc);
     if (!(f >= 0.0)) return 0;
     return f >= (double)nc ? nc - 1 : (int)f;
 }

@@ -349,3 +349,19 @@ def test_explicit_rows_of_every_length_are_sorted(gpu):
     p[flip] = p[flip, ::-1]
     ar.load_pairs(torch.from_numpy(np.ascontiguousarray(p)))
     _check_list_rows(ar, want)
+
+
+@pytest.mark.parametrize("n,ratio", [(1000, 3.05), (1000, 3.6), (1000, 4.5), (3000, 5.5), (9000, 6.3)])
+def test_list_of_positions_off_the_box(gpu, n, ratio):
+    """Positions are accepted up to one wrap off the box (in [0, L), or moved and not folded back): the cells
+    hold their images in the box, so the rows are those of all pairs under the one-wrap predicate."""
+    import nepx
+    from nepx.configs import make_system
+    shape = nepx.get_shape("cube8")
+    L = ratio * (shape.cutoff + 0.5)
+    spec = make_system("cube8", n, n * shape.volume / L ** 3, seed=n, non_overlap=False)
+    ar = nepx.Arena([spec], shape, (11, 6, 4), None, device=gpu)
+    for x in (np.where(spec.x < 0, spec.x + spec.L, spec.x), spec.x + 0.6, spec.x - 0.4 * spec.L):
+        ar.set_configuration(x)
+        ar.build_list(True)
+        _check_list_rows(ar, O.brute_pairs(x, spec.L, spec.rc + spec.skin))
