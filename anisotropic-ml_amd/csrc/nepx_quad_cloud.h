@@ -113,20 +113,23 @@ __device__ __forceinline__ void quad_cloud_sums(const float* pts, const float* _
     for (int n = 0; n < NA; ++n)
 #pragma unroll
         for (int l = 0; l < LMAX; ++l) ga[n][l] = 0.f;
-    static_for<LC>([&](auto dc) {  // this lane's column of chunk d is slot 4d + q; a chunk spans two l at most
+    // This lane's column of chunk d is slot 4d + q; a chunk spans two l at most.  A lane adds to its slot's own l
+    // only: with a zero weight for the other, a square past FP32's range (large site weights) would be NaN there
+    // (the selects: 1,000,003 clouds of 12 sites, hypers 10 8 4, 152 -> 154 us).
+    static_for<LC>([&](auto dc) {
         constexpr int d = decltype(dc)::value, last = 4 * d + 3 < MS::N ? 4 * d + 3 : MS::N - 1;
         constexpr int lo = MS::l_of(4 * d), hi = MS::l_of(last);
         constexpr float w0 = MS::k2(4 * d), w1 = MS::k2(4 * d + 1), w2 = MS::k2(4 * d + 2), w3 = MS::k2(4 * d + 3);
         constexpr int up = MS::off(hi) - 4 * d;  // first lane of the upper l
         static_assert(hi <= lo + 1, "a chunk spans two l at most");
         const float kk = sel4(q, w0, w1, w2, w3);
-        const float klo = lo == hi || q < up ? kk : 0.f, khi = lo == hi || q < up ? 0.f : kk;
+        const bool below = lo == hi || q < up;
 #pragma unroll
         for (int n = 0; n < NA; ++n) {
             const float v = Af[n / 4][d][n % 4];
             const float v2 = v * v;
-            ga[n][lo - 1] += klo * v2;
-            if (lo != hi) ga[n][hi - 1] += khi * v2;
+            ga[n][lo - 1] += kk * (below ? v2 : 0.f);
+            if (lo != hi) ga[n][hi - 1] += kk * (below ? 0.f : v2);
         }
     });
 #pragma unroll

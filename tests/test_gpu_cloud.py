@@ -121,3 +121,26 @@ def test_featurised_rows_equal_the_device_rows(gpu, n):
         nep.chunk = chunk
         G = nep.get_g_fast()
         assert G.dtype == np.float32 and G.shape == (n, 121) and np.array_equal(G, want)
+
+
+@pytest.mark.parametrize("hyp,scale", [((11, 6, 4), 1e18), ((11, 6, 4), 1e19), ((10, 8, 4), 1e18), ((17, 6, 6), 1e16),
+                                       ((17, 6, 6), 1e17), ((10, 10, 10), 1e13), ((10, 10, 10), 1e14),
+                                       ((10, 10, 10), 1e15)])
+def test_cloud_descriptor_overflow_stays_in_its_entry(gpu, hyp, scale):
+    """Site weights so large that the squared sums of the high l leave FP32's range: those entries are
+    infinite, none is NaN, and the entries of the lower l are those of the FP64 oracle.  The largest square of
+    an entry is at most the entry over its smallest K_lm^2 = 2 / (2l)!."""
+    from math import factorial
+    from nepx import ops
+    rng = np.random.default_rng(3)
+    nrad, nang, lmax = hyp
+    X = rng.normal(0, 1.0, (40, 12, 3)).astype(np.float32)
+    w = (scale * rng.uniform(0.5, 2.0, 12)).astype(np.float32)
+    G = ops.cloud_descriptor(torch.from_numpy(X).to(gpu), *hyp, 6.0, weights=w).cpu().numpy()
+    G64 = O.descriptor(X.astype(np.float64), 6.0, *hyp, weights=w.astype(np.float64))
+    k2min = np.array([2.0 / factorial(2 * l) for l in range(1, lmax + 1)])
+    safe = np.concatenate([np.ones((40, nrad + 1), bool),
+                           (G64[:, nrad + 1:].reshape(40, nang + 1, lmax) / k2min < 1e38).reshape(40, -1)], 1)
+    assert not np.isnan(G).any() and np.isinf(G).any() and safe.any(axis=0).sum() > nrad + 1
+    assert np.isfinite(G[safe]).all()
+    assert np.abs(G[safe] - G64[safe]).max() <= 1e-5 * np.abs(G64[safe]).max()
