@@ -42,6 +42,9 @@ __device__ __forceinline__ void quad_cloud_sums(const float* pts, const float* _
                                                 float (&ga)[Cfg::NANG + 1][Cfg::LMAX], Done&& sites_done) {
     using Q = QuadCloud<Cfg>;
     constexpr int NC = Q::NC, NA = Q::NA, LC = (MS::N + 3) / 4, LMAX = Cfg::LMAX;
+    // The set's first l, a compile-time constant: found at run time it leaves the sums below in scratch memory, walked by
+    // loops (hypers 10 10 10: 50 us a tile, 50,000 clouds of 12 sites 325 us against 55 us).
+    constexpr int FIRST = MS::l_of(0);
     v4f Af[NC][LC];
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -135,7 +138,7 @@ __device__ __forceinline__ void quad_cloud_sums(const float* pts, const float* _
 #pragma unroll
     for (int n = 0; n < NA; ++n)
 #pragma unroll
-        for (int l = MS::l_of(0) - 1; l < LMAX; ++l) ga[n][l] = quad_sum(ga[n][l]);  // zero below the set's first l
+        for (int l = FIRST - 1; l < LMAX; ++l) ga[n][l] = quad_sum(ga[n][l]);  // zero below the set's first l
 }
 
 // STAGED: the coordinates of the next tile go straight from memory to LDS (no registers) while this tile's

@@ -608,3 +608,17 @@ def test_isa_phase_counter_finds_every_site_trip():
     assert int(rows["forward"][1]) == 4 * 48 and int(rows["adjoint"][1]) == 3 * 84   # 4x4x1 products per trip
     total = int(rows["total per 16-pair wave iteration"][0])
     assert 2000 < total < 6000, total
+
+
+def test_no_kernel_keeps_an_array_in_scratch_memory():
+    """Private memory of every kernel in the built library, from the code objects' metadata: a few spilled
+    registers are accepted, an array that is indexed at run time (440 bytes of descriptor sums) is not."""
+    import re
+    from nepx import _lib
+    blob = open(_lib.LIB_PATH, "rb").read()
+    key = b"\xbb.private_segment_fixed_size"
+    kernels = re.findall(rb"\xa5\.name(?:[\xa0-\xbf]|\xd9.|\xda..)(_Z[ -~]+?)" + re.escape(key) +
+                         rb"([\x00-\x7f]|\xcc.|\xcd..)", blob, re.S)
+    assert len(kernels) == blob.count(key) > 50
+    size = {n.decode(): v[0] if len(v) == 1 else int.from_bytes(v[1:], "big") for n, v in kernels}
+    assert {n: v for n, v in size.items() if v > 160} == {}
