@@ -57,9 +57,10 @@ struct Reach {
     Mat3 R;
     float is, lx, ly, lz, hx, hy, hz;
 };
+// Below 1e-30 the division overflows or R has lost its bits to the end of FP32's range: NaN, which culls nothing.
 __device__ __forceinline__ Reach body_reach(const Mat3& R, const float4& q, const Box& b, float grow) {
     const float s = q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
-    return Reach{R, 1.f / s, s * b.lx - grow, s * b.ly - grow, s * b.lz - grow,
+    return Reach{R, s > 1e-30f ? 1.f / s : NAN, s * b.lx - grow, s * b.ly - grow, s * b.lz - grow,
                  s * b.hx + grow, s * b.hy + grow, s * b.hz + grow};
 }
 // False only for a point (relative to the body's centre) outside the grown box; a NaN stays in, so

@@ -163,3 +163,31 @@ def test_bead_cull_keeps_every_pair_in_reach(gpu, n_beads):
     for a, b, tol in ((got[:, 3], r["E"], 1e-5), (got[:, 0:3], r["F"], 1e-4), (got[:, 4:7], r["Ti"], 1e-4),
                       (got[:, 8:11], r["Tj"], 1e-4)):
         assert np.abs(a - b).max() <= tol * np.abs(b).max()
+
+
+@pytest.mark.parametrize("norm", [1e-14, 1e-15, 1e-16, 1e-18, 1e-20, 1e-22, 0.0])
+def test_bead_cull_with_vanishing_quaternions(gpu, norm):
+    """Quaternions of a norm near FP32's end shrink the bodies to their centres (the rotation formula scales
+    by the norm squared); every bead pair is then as far apart as the centres, and none is culled."""
+    from nepx import _lib, label
+    rng = np.random.default_rng(6)
+    P = 40
+    q = rng.normal(size=(2 * P, 4))
+    q = (q / np.linalg.norm(q, axis=1)[:, None] * norm).astype(np.float32)
+    pot = label.BeadPotential(device=gpu)
+    d = rng.normal(size=(P, 3))
+    r = np.linspace(0.05, 1.5, P) * pot.r0
+    t = (d / np.linalg.norm(d, axis=1)[:, None] * r[:, None]).astype(np.float32)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    qf, pi, pj = dev(q), dev(np.arange(P, dtype=np.int32)), dev(np.arange(P, 2 * P, dtype=np.int32))
+    pt = dev(np.concatenate([t, np.zeros((P, 1), np.float32)], 1))
+    out = torch.full((P * 12,), float("nan"), device=gpu)
+    n_dev = torch.tensor([P], dtype=torch.int32, device=gpu)
+    pot.pair_forces(_lib.ptr(qf), _lib.ptr(pi), _lib.ptr(pj), _lib.ptr(pt), _lib.ptr(n_dev), P, _lib.ptr(out))
+    got = out.view(P, 12).cpu().numpy()
+    t64 = t.astype(np.float64)
+    w = np.maximum(pot.r0 - np.linalg.norm(t64, axis=1), 0.0)
+    E = len(pot.beads) ** 2 * pot.eps * (w / pot.sigma) ** 2
+    assert np.count_nonzero(E) > 20 and np.abs(got[:, 3] - E).max() <= 1e-5 * E.max()
+    F = (-2.0 * len(pot.beads) ** 2 * pot.eps / pot.sigma ** 2 * w / np.linalg.norm(t64, axis=1))[:, None] * t64
+    assert np.abs(got[:, 0:3] - F).max() <= 1e-4 * np.abs(F).max()
