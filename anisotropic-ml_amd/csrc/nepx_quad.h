@@ -64,15 +64,15 @@ __device__ __forceinline__ float sel4(int q, float v0, float v1, float v2, float
     return q == 0 ? v0 : q == 1 ? v1 : q == 2 ? v2 : v3;
 }
 
-// Each block takes blockDim/4 consecutive pairs per iteration (16 per wave);
-// waves share nothing but the network weights, so the loop has no block barriers.
-// BLOCK threads at most; launches for few pairs use fewer (launch_fused_quad).
+// Each block takes BLOCK/4 consecutive pairs per iteration (16 per wave), or half as many on half its waves
+// while all pairs are few (launch_fused_quad); waves share nothing but the network weights, so the loop has no
+// block barriers.
 template <class Cfg, class N, int PREC, int ACT>
 __global__ __launch_bounds__(QuadCfg<Cfg>::BLOCK) __attribute__((
     amdgpu_waves_per_eu(QuadCfg<Cfg>::WAVES_PER_SIMD, QuadCfg<Cfg>::WAVES_PER_SIMD))) void k_fused_quad(
     nepx_pair_model m, const float* __restrict__ Wg, const void* __restrict__ Whg, float en_min, float scale,
     const float4* __restrict__ qf, const int32_t* __restrict__ pi, const int32_t* __restrict__ pj,
-    const float4* __restrict__ pt, const int32_t* __restrict__ np_dev, int64_t maxp, float clip,
+    const float4* __restrict__ pt, const int32_t* __restrict__ np_dev, int64_t maxp, int half_pairs, float clip,
     float* __restrict__ out, RevOut rv) {
     using Q = QuadCfg<Cfg>;
     static_assert(Q::OK, "shape not supported by the four-lane kernel");
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(QuadCfg<Cfg>::BLOCK) __attribute__((
     __shared__ __attribute__((aligned(16))) float wl[weight_lds_floats<N, PREC>()];
     const int P = n_pairs(np_dev, maxp);
     const int tag = rev_tag(rv);
-    const int per_block = blockDim.x >> 2;
+    const int per_block = P <= half_pairs ? Q::BLOCK / 8 : Q::BLOCK / 4;
     if ((int64_t)blockIdx.x * per_block >= P) return;  // no pairs (the grid is sized by the capacity)
     if (threadIdx.x == 0) {
 #pragma unroll
@@ -102,6 +102,7 @@ __global__ __launch_bounds__(QuadCfg<Cfg>::BLOCK) __attribute__((
     const void* WH;
     stage_net<N, PREC>(wl, Wg, Whg, W, WH);
     __syncthreads();
+    if ((int)(threadIdx.x >> 2) >= per_block) return;  // whole waves, past the last barrier
 
     const int lane = threadIdx.x & 63, q = lane & 3, wv = threadIdx.x >> 6, slot = lane >> 2;
     float* const xw = xch[wv];

@@ -10,13 +10,13 @@
 namespace nepx {
 
 template <class Cfg, class N, int PREC>
-static void launch_quad_p(const nepx_pair_model& m, const nepx_net* net, int grid, int block, float scale, const float* qf,
+static void launch_quad_p(const nepx_pair_model& m, const nepx_net* net, int grid, int half_pairs, float scale, const float* qf,
                           const int32_t* pair_i, const int32_t* pair_j, const float* pair_t, const int32_t* np_dev,
                           int64_t maxp, float clip, float* out, RevOut rv, void* stream) {
 #define NEPX_LAUNCH_QUAD(A)                                                                                      \
-    hipLaunchKernelGGL((k_fused_quad<Cfg, N, PREC, A>), dim3(grid), dim3(block), 0, as_stream(stream), m,         \
-                       net->w_packed, net->w_half, net->en_min, scale, (const float4*)qf, pair_i, pair_j,          \
-                       (const float4*)pair_t, np_dev, maxp, clip, out, rv)
+    hipLaunchKernelGGL((k_fused_quad<Cfg, N, PREC, A>), dim3(grid), dim3(QuadCfg<Cfg>::BLOCK), 0,                \
+                       as_stream(stream), m, net->w_packed, net->w_half, net->en_min, scale, (const float4*)qf,   \
+                       pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, half_pairs, clip, out, rv)
     if (net->act == NEPX_ACT_TANH) NEPX_LAUNCH_QUAD(NEPX_ACT_TANH);
     else if constexpr (PREC == NEPX_NET_F32 || PREC == NEPX_NET_F16X3) NEPX_LAUNCH_QUAD(NEPX_ACT_RELU);
 #undef NEPX_LAUNCH_QUAD
@@ -30,28 +30,31 @@ int launch_fused_quad(const nepx_pair_model& m, const nepx_net* net, int prec, i
         return NEPX_EUNSUP;
     } else {
         using Q = QuadCfg<Cfg>;
-        // Few pairs: with two waves per SIMD, half a block per CU while the capacity (about four times the pairs
-        // of a simulation's list) allows no more than four such rounds, so that the pairs spread over twice
-        // the CUs and a wave has its SIMD to itself (512 cubes, 4,800 pairs: 19.2 -> 14.7 us).
-        const int block = Q::WAVES_PER_SIMD == 2 && maxp <= (int64_t)4 * max_blocks * (Q::BLOCK / 8) ? Q::BLOCK / 2
-                                                                                                     : Q::BLOCK;
-        int64_t g = (maxp + block / 4 - 1) / (block / 4);
+        // Few pairs: with two waves per SIMD, half a block's waves take pairs while one round of half blocks, one
+        // a CU, holds them all: they spread over twice the CUs and a wave has its SIMD to itself (512 cubes,
+        // 4,800 pairs: 19.2 -> 14.7 us).  The kernel decides by the pair count, not the capacity: with half
+        // blocks up to some capacity, calls whose capacity is their count took two rounds where whole blocks
+        // take one (cube8, 17,000 pairs 24.5 us against 19.8, 50,000 pairs 44.8 against 35.0).
+        constexpr int HALF = Q::WAVES_PER_SIMD == 2 ? Q::BLOCK / 8 : 0;
+        const int half_pairs = device_cus() * HALF;
+        const int64_t least = HALF ? HALF : Q::BLOCK / 4;  // pairs a block takes at least
+        const int64_t g = (maxp + least - 1) / least;
         const int grid = (int)(g < 1 ? 1 : g > max_blocks ? max_blocks : g);
         switch (prec) {
             case NEPX_NET_F16X3:
-                launch_quad_p<Cfg, N, NEPX_NET_F16X3>(m, net, grid, block, scale, qf, pair_i, pair_j, pair_t, np_dev, maxp,
+                launch_quad_p<Cfg, N, NEPX_NET_F16X3>(m, net, grid, half_pairs, scale, qf, pair_i, pair_j, pair_t, np_dev, maxp,
                                                        clip, out, rv, stream);
                 break;
             case NEPX_NET_BF16:
-                launch_quad_p<Cfg, N, NEPX_NET_BF16>(m, net, grid, block, scale, qf, pair_i, pair_j, pair_t, np_dev, maxp,
+                launch_quad_p<Cfg, N, NEPX_NET_BF16>(m, net, grid, half_pairs, scale, qf, pair_i, pair_j, pair_t, np_dev, maxp,
                                                       clip, out, rv, stream);
                 break;
             case NEPX_NET_BF16X3:
-                launch_quad_p<Cfg, N, NEPX_NET_BF16X3>(m, net, grid, block, scale, qf, pair_i, pair_j, pair_t, np_dev,
+                launch_quad_p<Cfg, N, NEPX_NET_BF16X3>(m, net, grid, half_pairs, scale, qf, pair_i, pair_j, pair_t, np_dev,
                                                         maxp, clip, out, rv, stream);
                 break;
             default:
-                launch_quad_p<Cfg, N, NEPX_NET_F32>(m, net, grid, block, scale, qf, pair_i, pair_j, pair_t, np_dev, maxp,
+                launch_quad_p<Cfg, N, NEPX_NET_F32>(m, net, grid, half_pairs, scale, qf, pair_i, pair_j, pair_t, np_dev, maxp,
                                                      clip, out, rv, stream);
         }
         NEPX_LAUNCH_CHECK();

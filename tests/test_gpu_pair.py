@@ -315,6 +315,40 @@ def test_fused_few_pairs_launch_equals_wide_launch(gpu, shape_name, n_pairs):
     assert torch.equal(res[0], res[1])
 
 
+@pytest.mark.parametrize("shape_name", ["cube8", "tet10"])
+def test_fused_block_does_not_depend_on_the_capacity(gpu, shape_name):
+    """Whether whole or half blocks take the pairs is decided by their count on the device: a capacity equal to
+    the count launches the same blocks as a larger one, and counts on both sides of one half block a CU give
+    the same bits for every capacity."""
+    import ctypes as C
+    import nepx
+    from graph_util import kernel_launches
+    from nepx import _lib
+    shape, _, T = _inputs(gpu, shape_name, n_pairs=40000, seed=22)
+    model = nepx.make_pair_model(shape, (11, 6, 4))
+    net = nepx.EnergyNet.random(40, [64, 64], seed=7, device=gpu)
+    cn = net.cstruct()
+    half = 64 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    out, n_dev = torch.empty((40000, 12), device=gpu), torch.zeros(1, dtype=torch.int32, device=gpu)
+
+    def run(maxp, stream=None):
+        _lib.check(_lib.lib.nepx_pair_fused(C.byref(model), C.byref(cn), _lib.ptr(T["qf"]), _lib.ptr(T["pi"]),
+                                            _lib.ptr(T["pj"]), _lib.ptr(T["pt"]), _lib.ptr(n_dev), maxp, 100.0,
+                                            _lib.ptr(out), _lib.stream_handle(stream)), "nepx_pair_fused")
+
+    shapes = {tuple(kernel_launches(lambda s: run(m, s))) for m in (17000, 40000, 60000, 200000)}
+    assert len(shapes) == 1
+    n_dev.fill_(40000)
+    run(40000)
+    want = out.clone()
+    for n in (half - 1, half, half + 1, 2 * half, 2 * half + 1):
+        for maxp in (n, 100000):
+            out.fill_(float("nan"))
+            n_dev.fill_(n)
+            run(maxp)
+            assert torch.equal(out[:n], want[:n]) and torch.isnan(out[n:]).all()
+
+
 @pytest.mark.parametrize("precision", ["f32", "f16x3", "bf16x3", "bf16"])
 @pytest.mark.parametrize("shape_name,hyp,widths", [("tet10", (11, 6, 4), [64, 64]), ("cube8", (11, 6, 4), [64, 64]),
                                                    ("cyl12", (17, 6, 6), [128, 128])])
