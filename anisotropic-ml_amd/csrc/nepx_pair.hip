@@ -63,16 +63,18 @@ __global__ __launch_bounds__(kBlock) void k_desc_fwd(nepx_pair_model m, const fl
     }
 }
 
+// few: up to this many pairs are left to the four-lane kernel launched with it (0: this one takes them all).
 template <class Cfg>
 __global__ __launch_bounds__(kBlock) NEPX_ADJ_ATTR void k_adjoint(nepx_pair_model m, const float4* __restrict__ qf,
                                                     const int32_t* __restrict__ pi,
                                                     const int32_t* __restrict__ pj,
                                                     const float4* __restrict__ pt,
-                                                    const int32_t* __restrict__ np_dev, int64_t maxp,
+                                                    const int32_t* __restrict__ np_dev, int64_t maxp, int few,
                                                     const float* __restrict__ dEdG,
                                                     const float* __restrict__ E, float clip,
                                                     float* __restrict__ out) {
     const int P = n_pairs(np_dev, maxp);
+    if (P <= few) return;
     for (int idx = blockIdx.x * kBlock + threadIdx.x; idx < P; idx += gridDim.x * kBlock) {
         float4 qi, qj, t;
         load_pair(qf, pi, pj, pt, idx, qi, qj, t);
@@ -709,28 +711,47 @@ static void launch_desc_fwd(const nepx_pair_model& m, const float* qf, const int
                        (const float4*)qf, pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, G);
 }
 
+// Hypers 10 8 4, four sites: many pairs keep one lane per pair, whose two passes cost less than the four lanes'
+// exchange once the chip is full (two rounds of its lanes).  One lane -> four, one call of that many pairs:
+//   4 sites: 100,001 pairs 52 -> 45 us, 200,000 100 -> 98, 260,000 106 -> 121, 500,000 198 -> 228, 1,000,000 382 -> 450
+//   6 sites: 100,001 pairs 71 -> 54 us, 200,000 139 -> 119, 260,000 143 -> 148, 350,000 207 -> 198, 1,000,000 531 -> 550
+// Six sites lie within 4 % either way beyond the line and stay on four lanes, as do hypers 10 10 10 (eight
+// passes), which gain at every size.  The count decides, on the device: a capacity past the line launches
+// both kernels, and one of them leaves at once (3 us; by the capacity alone, 70,000 pairs in a list of
+// 280,000 slots would take 50 us in place of 34).
+template <class T>
+constexpr bool one_lane_for_many() { return adjoint_on_quads<T>() && T::LMAX <= 4 && T::NS <= 4; }
+template <class T>
+static int quad_adjoint_pairs() {
+    return one_lane_for_many<T>() ? 14 * 64 * device_cus() : INT32_MAX;
+}
+
 template <class T>
 static int launch_adjoint(const nepx_pair_model& m, const float* qf, const int32_t* pair_i, const int32_t* pair_j,
                           const float* pair_t, const int32_t* np_dev, int64_t maxp, const float* dEdG,
                           const float* E, float clip, float* out, void* stream) {
+    int few = 0;
     if constexpr (adjoint_on_quads<T>()) {
-        return launch_adjoint_quad<T>(m, (int)(device_cus() * (int64_t)tuning().pair_blocks_per_cu), qf, pair_i,
-                                      pair_j, pair_t, np_dev, maxp, dEdG, E, clip, out, stream);
-    } else {
-        if constexpr (!T::ONE_PASS) {
-            if (by_passes<T>(maxp)) {
-                hipLaunchKernelGGL(k_adjoint_passes<T>, dim3(pass_grid(maxp)), dim3(64 * pass_waves<T>()), 0,
-                                   as_stream(stream), m, (const float4*)qf, pair_i, pair_j, (const float4*)pair_t,
-                                   np_dev, maxp, dEdG, E, clip, out);
-                NEPX_LAUNCH_CHECK();
-                return NEPX_OK;
-            }
+        few = quad_adjoint_pairs<T>();
+        const int rc = launch_adjoint_quad<T>(m, (int)(device_cus() * (int64_t)tuning().pair_blocks_per_cu), qf, pair_i,
+                                              pair_j, pair_t, np_dev, maxp, few, dEdG, E, clip, out, stream);
+        if (rc || maxp <= few) return rc;
+    } else if constexpr (!T::ONE_PASS) {
+        if (by_passes<T>(maxp)) {
+            hipLaunchKernelGGL(k_adjoint_passes<T>, dim3(pass_grid(maxp)), dim3(64 * pass_waves<T>()), 0,
+                               as_stream(stream), m, (const float4*)qf, pair_i, pair_j, (const float4*)pair_t,
+                               np_dev, maxp, dEdG, E, clip, out);
+            NEPX_LAUNCH_CHECK();
+            return NEPX_OK;
         }
-        hipLaunchKernelGGL(k_adjoint<T>, dim3(grid_for(maxp, kBlock)), dim3(kBlock), 0, as_stream(stream), m,
-                           (const float4*)qf, pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, dEdG, E, clip, out);
-        NEPX_LAUNCH_CHECK();
-        return NEPX_OK;
     }
+    if constexpr (!adjoint_on_quads<T>() || one_lane_for_many<T>()) {
+        hipLaunchKernelGGL(k_adjoint<T>, dim3(grid_for(maxp, kBlock)), dim3(kBlock), 0, as_stream(stream), m,
+                           (const float4*)qf, pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, few, dEdG, E, clip,
+                           out);
+        NEPX_LAUNCH_CHECK();
+    }
+    return NEPX_OK;
 }
 
 static bool desc_supported(const nepx_pair_model* m) {

@@ -203,7 +203,8 @@ struct QuadCfg {
     static constexpr int BLOCK = 256 * WAVES_PER_SIMD;
 };
 
-// Shapes whose adjoint runs four lanes per pair (nepx_quad_adjoint.h): those without a fused kernel.  The
+// Shapes whose adjoint runs four lanes per pair (nepx_quad_adjoint.h), for up to `most` pairs: those without a
+// fused kernel.  The
 // shapes with one keep k_adjoint, whose results equal the one-lane fused kernel's bit for bit.
 template <class Cfg>
 constexpr bool adjoint_on_quads() {
@@ -212,7 +213,7 @@ constexpr bool adjoint_on_quads() {
 }
 template <class Cfg>
 int launch_adjoint_quad(const nepx_pair_model& m, int max_blocks, const float* qf, const int32_t* pair_i,
-                        const int32_t* pair_j, const float* pair_t, const int32_t* np_dev, int64_t maxp,
+                        const int32_t* pair_j, const float* pair_t, const int32_t* np_dev, int64_t maxp, int most,
                         const float* dEdG, const float* E, float clip, float* out, void* stream);
 
 // Hypers with a cloud descriptor kernel.

@@ -73,20 +73,21 @@ NEPX_QUAD_INSTANCE(CfgCyl12, Net60x128)
 
 template <class Cfg>
 int launch_adjoint_quad(const nepx_pair_model& m, int max_blocks, const float* qf, const int32_t* pair_i,
-                        const int32_t* pair_j, const float* pair_t, const int32_t* np_dev, int64_t maxp,
+                        const int32_t* pair_j, const float* pair_t, const int32_t* np_dev, int64_t maxp, int most,
                         const float* dEdG, const float* E, float clip, float* out, void* stream) {
     static_assert(QuadAdj<Cfg>::OK, "whole quads of sites");
     const int64_t tiles = (maxp + 15) / 16;
     const int grid = (int)(tiles < max_blocks ? tiles : max_blocks);
     hipLaunchKernelGGL(k_adjoint_quad<Cfg>, dim3(grid), dim3(QuadAdj<Cfg>::BLOCK), 0, as_stream(stream), m,
-                       (const float4*)qf, pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, dEdG, E, clip, out);
+                       (const float4*)qf, pair_i, pair_j, (const float4*)pair_t, np_dev, maxp, most, dEdG, E, clip,
+                       out);
     NEPX_LAUNCH_CHECK();
     return NEPX_OK;
 }
 #define NEPX_QUAD_ADJOINT(T)                                                                                  \
     template int launch_adjoint_quad<T>(const nepx_pair_model&, int, const float*, const int32_t*,            \
-                                        const int32_t*, const float*, const int32_t*, int64_t, const float*,  \
-                                        const float*, float, float*, void*);
+                                        const int32_t*, const float*, const int32_t*, int64_t, int,           \
+                                        const float*, const float*, float, float*, void*);
 NEPX_QUAD_ADJOINT(CfgCubeV2)
 NEPX_QUAD_ADJOINT(CfgThV1)
 NEPX_QUAD_ADJOINT(CfgCubeV2L10)

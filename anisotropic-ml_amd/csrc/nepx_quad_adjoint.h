@@ -250,7 +250,7 @@ __device__ __forceinline__ void quad_adjoint_sums(float inv_rn, const QuadSites<
 template <class Cfg>
 __global__ __launch_bounds__((QuadAdj<Cfg>::BLOCK)) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adjoint_quad(
     nepx_pair_model m, const float4* __restrict__ qf, const int32_t* __restrict__ pi, const int32_t* __restrict__ pj,
-    const float4* __restrict__ pt, const int32_t* __restrict__ np_dev, int64_t maxp,
+    const float4* __restrict__ pt, const int32_t* __restrict__ np_dev, int64_t maxp, int most,
     const float* __restrict__ dEdG, const float* __restrict__ E, float clip, float* __restrict__ out) {
     using Q = QuadAdj<Cfg>;
     using MG = typename Q::MG;
@@ -261,7 +261,8 @@ __global__ __launch_bounds__((QuadAdj<Cfg>::BLOCK)) __attribute__((amdgpu_waves_
     __shared__ float part[COUNT][12][PW];
     __shared__ float4 stab[Cfg::ND];
     const int P = n_pairs(np_dev, maxp);
-    if ((int64_t)blockIdx.x * PW >= P) return;  // the grid is sized by the capacity
+    // the grid is sized by the capacity; more than `most` pairs go one to a lane (k_adjoint)
+    if ((int64_t)blockIdx.x * PW >= P || P > most) return;
     if (threadIdx.x < Cfg::ND) {
         const int k = threadIdx.x % Cfg::NS;
         stab[threadIdx.x] = make_float4(m.sites[3 * k], m.sites[3 * k + 1], m.sites[3 * k + 2], 0.f);

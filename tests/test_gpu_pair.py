@@ -223,6 +223,52 @@ def test_quad_adjoint_tile_edges(gpu, shape_name, hyp, n_pairs):
         assert torch.equal(part[:n_pairs - 3], out[:n_pairs - 3])
 
 
+@pytest.mark.parametrize("shape_name", ["th_v1"])
+def test_adjoint_of_many_pairs_keeps_one_lane_per_pair(gpu, shape_name):
+    """Hypers 10 8 4, four sites: four lanes per pair up to 896 pairs a CU, one lane per pair beyond, by the count.  Counts on
+    both sides of the line, within a larger capacity and equal to it: the rows are those of the one or the
+    other kernel, match the FP64 oracle, and nothing is written past the last pair."""
+    import ctypes as C
+    import nepx
+    from graph_util import kernel_launches
+    from nepx import _lib
+    hyp = (10, 8, 4)
+    line = 896 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    n = line + 300
+    shape, (q, i, j, t), T = _inputs(gpu, shape_name, n_pairs=n, seed=17)
+    model = nepx.make_pair_model(shape, hyp)
+    g = torch.Generator(device=gpu).manual_seed(18)
+    dG = torch.randn((n, nepx.n_descriptor(*hyp)), generator=g, device=gpu)
+    n_dev, out = torch.zeros(1, dtype=torch.int32, device=gpu), torch.empty((n, 12), device=gpu)
+
+    def run(maxp, stream=None):
+        _lib.check(_lib.lib.nepx_descriptor_adjoint(
+            C.byref(model), _lib.ptr(T["qf"]), _lib.ptr(T["pi"]), _lib.ptr(T["pj"]), _lib.ptr(T["pt"]),
+            _lib.ptr(n_dev), maxp, _lib.ptr(dG), None, 0.0, _lib.ptr(out), _lib.stream_handle(stream)),
+            "nepx_descriptor_adjoint")
+
+    assert [b[0] for _, b in kernel_launches(lambda s: run(line, s))] == [128]
+    assert [b[0] for _, b in kernel_launches(lambda s: run(line + 1, s))] == [128, 256]
+    tail = slice(line - 300, line - 1)
+    clouds = oracle_clouds(q, i[tail], j[tail], t[tail], shape.sites)
+    gp = O.descriptor_grad(clouds, dG[tail].cpu().numpy().astype(np.float64), shape.nep_cutoff, *hyp)
+    Ns = shape.n_sites
+    arm_j = clouds[:, Ns:] - t[tail].astype(np.float64)[:, None, :]
+    want = np.concatenate([-gp[:, :Ns].sum(1), np.cross(clouds[:, :Ns], -gp[:, :Ns]).sum(1),
+                           np.cross(arm_j, -gp[:, Ns:]).sum(1)], 1)
+    rows = {}
+    for count in (line - 1, line, line + 1, n):
+        for maxp in (count, 4 * n):
+            out.fill_(float("nan"))
+            n_dev.fill_(count)
+            run(maxp)
+            assert torch.isfinite(out[:count]).all() and torch.isnan(out[count:]).all()
+            got = out[tail].cpu().numpy()
+            for a, b in ((0, 0), (4, 3), (8, 6)):
+                assert normwise_rel(got[:, a:a + 3], want[:, b:b + 3]) < 1e-4
+            assert np.array_equal(rows.setdefault(count > line, got), got)
+
+
 @pytest.mark.parametrize("shape_name,hyp", CASES)
 def test_pass_kernels_equal_pair_kernels(gpu, shape_name, hyp):
     """Few pairs of a multi-pass shape run their l-range passes on separate waves (descriptor and
