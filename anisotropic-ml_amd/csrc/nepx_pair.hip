@@ -6,7 +6,7 @@
 
 namespace nepx {
 
-// Descriptor row of one pair, one pass over the sites per l range.
+// Descriptor row of one pair (or cloud), one pass over the sites per l range.
 template <class Cfg, class Sites, class Row>
 __device__ __forceinline__ void desc_forward_sites(const Sites& sites, Row&& G) {
     float grad[Cfg::NRAD + 1];
@@ -1201,6 +1201,91 @@ extern "C" int nepx_fd_forces(const float* E_rows, int64_t P, float dx, float dt
     return NEPX_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Descriptors of site clouds, one cloud per lane (four lanes: nepx_quad_cloud.h): nd points of a cloud (xyz
+// interleaved) about their centroid, optional per-point weights.
+struct CloudSites {
+    const float* __restrict__ pts;
+    const float* __restrict__ w;
+    int nd;
+    float cx, cy, cz, inv_rn;
+    __device__ __forceinline__ CloudSites(const float* pts_, const float* w_, int nd_, float inv_rn_)
+        : pts(pts_), w(w_), nd(nd_), inv_rn(inv_rn_) {
+        float sx = 0.f, sy = 0.f, sz = 0.f;
+        for (int a = 0; a < nd; ++a) {
+            sx += pts[3 * a];
+            sy += pts[3 * a + 1];
+            sz += pts[3 * a + 2];
+        }
+        const float inv = 1.f / (float)nd;
+        cx = sx * inv;
+        cy = sy * inv;
+        cz = sz * inv;
+    }
+    template <class S, class B>
+    __device__ __forceinline__ void visit(S&& site, B&& body_done) const {
+#pragma unroll 1
+        for (int a = 0; a < nd; ++a) {
+            SiteGeo s;
+            s.ax = s.ay = s.az = 0.f;
+            const float rx = pts[3 * a] - cx, ry = pts[3 * a + 1] - cy, rz = pts[3 * a + 2] - cz;
+            const float r2 = rx * rx + ry * ry + rz * rz;
+            s.ir = __builtin_amdgcn_rsqf(r2);
+            s.r = r2 * s.ir;
+            s.ux = rx * s.ir;
+            s.uy = ry * s.ir;
+            s.uz = rz * s.ir;
+            s.rho = s.r * inv_rn;
+            site(s, w ? w[a] : 1.f);
+        }
+        body_done(0);
+    }
+};
+
+template <class Cfg>
+__global__ __launch_bounds__(kBlock) void k_cloud_desc(const float* __restrict__ clouds, int64_t P, int nd,
+                                                       const float* __restrict__ w, float r_nep,
+                                                       float* __restrict__ G) {
+    for (int64_t idx = blockIdx.x * (int64_t)kBlock + threadIdx.x; idx < P; idx += (int64_t)gridDim.x * kBlock) {
+        const CloudSites sites(clouds + idx * 3 * (int64_t)nd, w, nd, 1.f / r_nep);
+        if constexpr (Cfg::ONE_PASS) {
+            float Gr[Cfg::D];
+            desc_forward_sites<Cfg>(sites, Gr);
+            store_row<Cfg>(G + idx * Cfg::D, Gr);
+        } else {
+            desc_forward_sites<Cfg>(sites, G + idx * Cfg::D);
+        }
+    }
+}
+
+// Many clouds of 1, 2, 5 or 6 sites take one lane each where the rows are seven n wide: a quad's last trip is
+// then half idle, and closing a tile costs more than the sites.  One lane -> four lanes per cloud:
+//   hypers 11 6 4, 1,000,000 clouds: 1 site 57 -> 64 us, 2 sites 62 -> 66, 3 sites 67 -> 66, 4 sites 72 -> 66,
+//     5 sites 79 -> 92, 6 sites 85 -> 94, 8 sites 99 -> 97; 60,000 clouds: 5 sites 9.4 -> 9.3, 6 sites 10.0 -> 9.4
+//   hypers 17 6 6, 1,000,000 clouds: 1 site 94 -> 127 us, 2 sites 107 -> 128, 3 sites 122 -> 126, 4 sites
+//     135 -> 127, 5 sites 151 -> 174, 6 sites 162 -> 174, 8 sites 202 -> 176; 100,000 clouds: 5 sites 20.5 -> 22.8;
+//     60,000 clouds: 5 sites 15.8 -> 15.1, 6 sites 17.4 -> 15.2
+// From seven sites on, and with the other hypers, four lanes gain at every size.
+template <class Cfg>
+constexpr bool few_sites_on_lanes() { return Cfg::NANG == 6; }
+static bool one_lane_clouds(int64_t n_clouds, int n_sites) {
+    return n_sites <= 6 && (n_sites - 1) % 4 < 2 && n_clouds >= 320 * (int64_t)device_cus();
+}
+
+template <class Cfg>
+static int launch_clouds(const float* clouds, int64_t n_clouds, int n_sites, const float* site_w, float r_nep,
+                         float* G, void* stream) {
+    if constexpr (few_sites_on_lanes<Cfg>()) {
+        if (one_lane_clouds(n_clouds, n_sites)) {
+            hipLaunchKernelGGL(k_cloud_desc<Cfg>, dim3(grid_for(n_clouds, kBlock)), dim3(kBlock), 0,
+                               as_stream(stream), clouds, n_clouds, n_sites, site_w, r_nep, G);
+            NEPX_LAUNCH_CHECK();
+            return NEPX_OK;
+        }
+    }
+    return launch_cloud_quad<Cfg>(clouds, n_clouds, n_sites, site_w, r_nep, G, stream);
+}
+
 extern "C" int nepx_cloud_descriptor(const float* clouds, int64_t n_clouds, int32_t n_sites, const float* site_w,
                                      int32_t nrad, int32_t nang, int32_t lmax, float r_nep, float* G,
                                      void* stream) {
@@ -1211,8 +1296,7 @@ extern "C" int nepx_cloud_descriptor(const float* clouds, int64_t n_clouds, int3
     NEPX_REQUIRE(clouds && G, NEPX_EINVAL, "null buffer");
 #define X(a, b, c)                                                                                       \
     if (nrad == a && nang == b && lmax == c)                                                             \
-        return launch_cloud_quad<DescCfg<1, a, b, c>>(clouds, n_clouds, (int)n_sites, site_w, r_nep, G,  \
-                                                      stream);
+        return launch_clouds<DescCfg<1, a, b, c>>(clouds, n_clouds, (int)n_sites, site_w, r_nep, G, stream);
     NEPX_CLOUD_CASES(X)
 #undef X
     set_error("no cloud descriptor kernel for hypers (%d, %d, %d)", nrad, nang, lmax);

@@ -144,3 +144,36 @@ def test_cloud_descriptor_overflow_stays_in_its_entry(gpu, hyp, scale):
     assert not np.isnan(G).any() and np.isinf(G).any() and safe.any(axis=0).sum() > nrad + 1
     assert np.isfinite(G[safe]).all()
     assert np.abs(G[safe] - G64[safe]).max() <= 1e-5 * np.abs(G64[safe]).max()
+
+
+@pytest.mark.parametrize("hyp", [(11, 6, 4), (10, 8, 4), (17, 6, 6), (10, 10, 10)])
+@pytest.mark.parametrize("nd", [2, 3, 4, 5, 6, 7])
+def test_many_clouds_of_few_sites(gpu, hyp, nd):
+    """1, 2, 5 and 6 sites with seven-wide rows, from 320 clouds a CU on: one lane per cloud, blocks of 256 (four
+    lanes: 64 or 256).  Counts on both sides of the line against the FP64 oracle, in a row block that is
+    4 bytes off."""
+    import nepx
+    from graph_util import kernel_launches
+    from nepx import _lib
+    line = 320 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    D = nepx.n_descriptor(*hyp)
+    g = torch.Generator(device=gpu).manual_seed(nd)
+    X = torch.randn((line + 70, nd, 3), generator=g, device=gpu)
+    w = torch.from_numpy(np.random.default_rng(nd).uniform(0.5, 2.0, nd).astype(np.float32)).to(gpu)
+    buf = torch.empty((line + 70) * D + 8, device=gpu)
+    blocks = []
+    for P in (line - 1, line, line + 70):
+        def run(stream=None):
+            _lib.check(_lib.lib.nepx_cloud_descriptor(_lib.ptr(X), P, nd, _lib.ptr(w), *hyp, 6.0,
+                                                      buf.data_ptr() + 4, _lib.stream_handle(stream)),
+                       "nepx_cloud_descriptor")
+        buf.fill_(float("nan"))
+        run()
+        G = buf[1:1 + P * D].view(P, D)
+        assert torch.isnan(buf[0]) and torch.isnan(buf[1 + P * D:]).all() and torch.isfinite(G).all()
+        pick = torch.cat([torch.arange(30), torch.arange(P - 90, P)])
+        G64 = O.descriptor(X[pick].cpu().numpy().astype(np.float64), 6.0, *hyp, weights=w.cpu().numpy().astype(np.float64))
+        assert _rowwise(G[pick].cpu().numpy(), G64) < 1e-5
+        blocks.append(kernel_launches(run)[0][1][0])
+    four = 256 if hyp[2] == 10 else 64
+    assert blocks == [four] + [256 if hyp[1] == 6 and nd in (2, 5, 6) else four] * 2
