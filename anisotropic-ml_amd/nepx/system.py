@@ -25,15 +25,37 @@ def _align(n, b=BLOCK):
     return (n + b - 1) // b * b
 
 
-def _cells_per_side(n, L, r_list):
-    """Cells per side of the list build (0: all pairs).  Cells of side r_list or more where they hold few
-    particles; with 8 or more in such a cell, cells of half that side (a particle then reaches 5^3 of them):
-    they cover 15.6 instead of 27 r_list^3 of candidates, while few of their walks come out short."""
-    nc = int(math.floor(L / r_list))
-    fine = int(math.floor(2.0 * L / r_list))
-    if fine >= 5 and n >= 8 * max(nc, 1) ** 3:
-        return fine
-    return nc if nc >= 3 else 0
+WIDE_GROUPS = 8192     # particles of an arena up to which the list build gives each a wave, beyond 16 lanes
+
+
+def _walk_rounds(n, nc, reach, lanes):
+    """Rounds of `lanes` candidates a particle's walk takes over the cells within `reach` of its own: the entries of
+    span^2 columns, and one and a half rounds for each run of a column (its start and its partly filled
+    end); a column that wraps is two runs."""
+    span = min(2 * reach + 1, nc)
+    runs = 1.0 + (span - 1) / nc if span < nc else 1.0
+    return span * span * (n / nc ** 3 * span / lanes + 1.5 * runs)
+
+
+def _cells_per_side(n, L, r_list, n_arena):
+    """Cells per side of the list build of n particles (0: all pairs), in an arena of n_arena.
+
+    Cells of side r_list (27 around a particle) or of half that (125 of an eighth the volume, 15.6 instead of 27
+    r_list^3 of candidates in 25 instead of 9 columns): the ones with the shorter walk.  Half-size cells pay
+    where columns are long, from about 30 particles per r_list^3 with 16 lanes and 100 with 64, and in boxes of
+    3.5 r_list or more.  Forced builds, full-size -> half-size cells, per r_list^3, box side in r_list, bodies:
+      16 lanes: 100 in 6.2, 23,832: 690 -> 592 us; 64 in 6.2, 15,252: 339 -> 294; 32 in 4.3, 8 x 2,544: 243 -> 236;
+                24 in 6.2, 3 x 5,719: 194 -> 198; 13 in 3.05, 40 x 365: 130 -> 178; 6 in 6.2, 42 x 1,429: 225 -> 385
+      64 lanes: 100 in 3.6, 4,665: 181 -> 167 us; 64 in 4.3, 5,088: 130 -> 140; 13 in 3.05, 16 x 365: 82 -> 162;
+                12 in 2.55 (all pairs), 16 x 200: 40 -> 79
+    """
+    lanes = 64 if n_arena <= WIDE_GROUPS else 16
+    nc, fine = int(math.floor(L / r_list)), int(math.floor(2.0 * L / r_list))
+    full = nc if nc >= 3 else 0
+    if fine < 5:
+        return full
+    rounds = _walk_rounds(n, full, 1, lanes) if full else n / lanes + 1.5
+    return fine if _walk_rounds(n, fine, 2, lanes) < rounds else full
 
 
 class SystemSpec:
@@ -111,7 +133,7 @@ class Arena:
             r_list = sp.rc + sp.skin
             if sp.L < 2.0 * sp.rc:
                 raise ValueError(f"box {sp.L} smaller than twice the cutoff {sp.rc}")
-            nc = _cells_per_side(sp.n, sp.L, r_list)
+            nc = _cells_per_side(sp.n, sp.L, r_list, self.n)
             r = rec[k]
             r["L"], r["kT"], r["dt"], r["tau"] = sp.L, sp.kT, sp.dt, sp.tau
             r["ndof"], r["rndof"] = sp.ndof, sp.rndof

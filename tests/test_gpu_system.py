@@ -365,3 +365,23 @@ def test_list_of_positions_off_the_box(gpu, n, ratio):
         ar.set_configuration(x)
         ar.build_list(True)
         _check_list_rows(ar, O.brute_pairs(x, spec.L, spec.rc + spec.skin))
+
+
+@pytest.mark.parametrize("full_size", [True, False])
+@pytest.mark.parametrize("n,copies,ratio", [(200, 4, 2.55), (200, 4, 2.95), (300, 4, 3.05), (300, 4, 3.45), (365, 3, 3.55),
+                                            (300, 31, 2.6), (365, 23, 3.2), (700, 13, 4.3)])
+def test_list_of_batched_small_boxes(gpu, monkeypatch, n, copies, ratio, full_size):
+    """Boxes of 2.5 to 4.5 list radii batched past the one-block build, on 64 and on 16 lanes: all pairs or
+    full-size cells, and half-size cells (5 a side: the walk covers the box; 6 to 8: columns that wrap)."""
+    import nepx
+    from nepx import system
+    from nepx.configs import make_system
+    shape = nepx.get_shape("cube8")
+    r = shape.cutoff + 0.5
+    L = ratio * r
+    cells = int(ratio) if full_size else int(2 * ratio)
+    monkeypatch.setattr(system, "_cells_per_side", lambda *a: cells if cells >= 3 else 0)
+    specs = [make_system("cube8", n, n * shape.volume / L ** 3, seed=k, non_overlap=False) for k in range(copies)]
+    ar = nepx.Arena(specs, shape, (11, 6, 4), None, device=gpu)
+    ar.build_list(True)
+    _check_list_rows(ar, np.concatenate([O.brute_pairs(s.x, s.L, r) + a for s, a in zip(specs, ar.starts)]))

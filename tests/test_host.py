@@ -622,3 +622,14 @@ def test_no_kernel_keeps_an_array_in_scratch_memory():
     assert len(kernels) == blob.count(key) > 50
     size = {n.decode(): v[0] if len(v) == 1 else int.from_bytes(v[1:], "big") for n, v in kernels}
     assert {n: v for n, v in size.items() if v > 160} == {}
+
+
+@pytest.mark.parametrize("n,ratio,n_arena,nc", [
+    # n bodies in a box of `ratio` list radii, in an arena of n_arena: the faster cells of measured builds
+    (64, 2.28, 256, 0), (200, 2.55, 4096, 0), (365, 2.95, 8192, 0), (843, 2.6, 24576, 0),
+    (365, 3.05, 8192, 3), (365, 3.55, 20480, 3), (1000, 4.5, 4096, 4), (1000, 4.5, 16384, 4), (1429, 6.2, 64512, 6),
+    (5719, 6.2, 17664, 6), (5088, 4.3, 5120, 4), (4097, 3.41, 4352, 3), (7950, 4.3, 8192, 4),
+    (4665, 3.6, 4864, 7), (4665, 3.6, 19456, 7), (15252, 6.2, 15360, 12), (48228, 9.1, 48384, 18), (32768, 6.8, 32768, 13)])
+def test_list_cells_take_the_shorter_walk(n, ratio, n_arena, nc):
+    from nepx.system import _cells_per_side
+    assert _cells_per_side(n, ratio * 3.0, 3.0, n_arena) == nc
