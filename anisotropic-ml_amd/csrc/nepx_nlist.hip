@@ -508,15 +508,18 @@ __global__ __launch_bounds__(kSortThreads) void k_rev_rows(nepx_nlist nl, int n)
 }
 
 // ---- whole build of a small list ------------------------------------------------
-// Up to kOneBuild particles in one block and one launch instead of nine: a build point of a captured run
-// costs 5 us instead of 41 when no rebuild is due, which most are not.  A rebuild costs 90 us at 512
-// particles, growing with n^2, against 55 us for the launches above, so the line lies where a rebuild and
-// the two or three build points that follow it cost the same either way.
+// A small list (n particles with padding) in one block and one launch instead of nine.  A build point that finds
+// no rebuild due costs 2 us instead of 14 (in a row of them in a graph), and most do; a rebuild costs more,
+// growing with n^2.  Rebuild in one block against the launches, cubes at packing 0.02 to 0.45: 256 particles
+// 27 to 47 us against 43 to 27, 384 49 to 74 against 39 to 47, 512 75 to 98 against 43 to 47, 640 115 to 156
+// against 44 to 48.  So a forced build, which always rebuilds, takes the block up to 256 particles (at 512,
+// energies and forces of one configuration: 204 to 226 us in one block, 171 to 175 with the launches), and a
+// conditional one up to 512, where three to four idle build points pay for a rebuild.
 // Every distance within a system is taken once (each wave: one particle against 64 later ones, the ballot
 // is a word of its row of the adjacency matrix in LDS; the words before the diagonal are then read off the
 // columns), and rows, reverse rows and slots are read off the matrix in order, so nothing is sorted or
 // searched.
-constexpr int kOneBuild = 640;
+constexpr int kOneBuild = 512, kOneBuildForced = 256;
 __global__ __launch_bounds__(kScanBlock) void k_build_one(nepx_state st, nepx_nlist nl, int force) {
     static_assert(kScanBlock >= kOneBuild && kOneBuild % 64 == 0, "one thread per particle");
     __shared__ uint64_t adj[kOneBuild * (kOneBuild / 64 | 1)];  // rows of an odd number of words: columns on distinct banks
@@ -973,7 +976,7 @@ extern "C" int nepx_nlist_build(nepx_state* st, nepx_nlist* nl, int32_t force, v
     NEPX_REQUIRE(((uintptr_t)nl->cell_pos & 31) == 0, NEPX_EINVAL, "cell_pos must be 32-byte aligned");
     hipStream_t s = as_stream(stream);
     const int n = st->n;
-    if (n <= kOneBuild && st->n_sys <= INT16_MAX) {
+    if (n <= (force ? kOneBuildForced : kOneBuild) && st->n_sys <= INT16_MAX) {
         hipLaunchKernelGGL(k_build_one, dim3(1), dim3(kScanBlock), 0, s, *st, *nl, force ? 1 : 0);
         NEPX_LAUNCH_CHECK();
         return NEPX_OK;

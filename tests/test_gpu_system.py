@@ -385,3 +385,47 @@ def test_list_of_batched_small_boxes(gpu, monkeypatch, n, copies, ratio, full_si
     ar = nepx.Arena(specs, shape, (11, 6, 4), None, device=gpu)
     ar.build_list(True)
     _check_list_rows(ar, np.concatenate([O.brute_pairs(s.x, s.L, r) + a for s, a in zip(specs, ar.starts)]))
+
+
+def test_small_list_build_launches(gpu):
+    """One block builds a list of up to 256 particles (with padding) when the build is forced and of up to 512 when
+    it is not, and the nine launches any other."""
+    import nepx
+    from graph_util import kernel_launches
+    from nepx.configs import make_system
+    spec = make_system("cube8", 700, 0.2, seed=1, non_overlap=False)
+    ar = nepx.Arena([spec], nepx.get_shape("cube8"), (11, 6, 4), None, device=gpu)
+    got = {}
+    for n in (1, 255, 256, 257, 511, 512, 513, 768):
+        ar.st.n = n
+        got[n] = tuple(len(kernel_launches(lambda s: ar.build_list(f, s))) for f in (True, False))
+    assert got == {n: (1 if n <= 256 else 9, 1 if n <= 512 else 9) for n in got}
+
+
+@pytest.mark.parametrize("force", [True, False])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 320, 447, 511, 512, 513, 640])
+def test_list_build_of_any_count(gpu, n, force):
+    """The C entry takes any particle count, not only the arena's whole blocks: ragged last words of the one-block
+    build's matrix and both sides of its limits, forced and when due, with the reverse-row entries, and
+    nothing written past the last row."""
+    import nepx
+    from nepx.configs import make_system
+    spec = make_system("cube8", 640, 0.3, seed=n, non_overlap=False)
+    ar = nepx.Arena([spec], nepx.get_shape("cube8"), (11, 6, 4), None, device=gpu, reverse_records=True)
+    for k in ("row_start", "rrow_start", "nbr", "slot_row", "rnbr", "rpos"):
+        ar.lt[k].fill_(-7)
+    ar.st.n = n
+    if not force:
+        ar.lt["flags"][0] = 1
+    ar.build_list(force)
+    want = O.brute_pairs(spec.x[:n], spec.L, spec.rc + spec.skin).reshape(-1, 2)
+    lt = {k: ar.lt[k].cpu().numpy() for k in ("nbr", "slot_row", "rnbr", "rpos", "row_start", "rrow_start", "flags")}
+    M = len(want)
+    assert lt["flags"][2] == M and list(lt["flags"][[0, 1, 7, 11]]) == [0, 0, 0, 0] and lt["flags"][4] == 1
+    assert np.array_equal(np.stack([lt["slot_row"][:M], lt["nbr"][:M]], 1), want)
+    assert np.array_equal(lt["row_start"][:n + 1], np.searchsorted(want[:, 0], np.arange(n + 1)))
+    order = np.lexsort((want[:, 0], want[:, 1]))
+    assert np.array_equal(lt["rnbr"][:M], order) and np.array_equal(lt["rnbr"][lt["rpos"][:M]], np.arange(M))
+    assert np.array_equal(lt["rrow_start"][:n + 1], np.searchsorted(want[order, 1], np.arange(n + 1)))
+    for k, m in (("row_start", n + 1), ("rrow_start", n + 1), ("nbr", M), ("slot_row", M), ("rnbr", M), ("rpos", M)):
+        assert (lt[k][m:] == -7).all(), k
