@@ -998,19 +998,20 @@ static int launch_ffnn(const nepx_net* net, int grid, float scale, int d, const 
 // The FP32 network runs on k_ffnn_spread where a block's copy of its operands does not fit in LDS (one
 // wave per tile would read them from L2 for every tile: 60 -> 128 x 2 at 20,000 rows 93 us against
 // 26, 121 -> 150 x 4 536 against 86), and, for the network that fits, up to four tiles per CU (too few
-// for a wave each; beyond, k_ffnn's copy in LDS is as fast); same results.
+// for a wave each; beyond, k_ffnn's copy in LDS is as fast); same results.  The grid is capped by
+// tuning().net_blocks_per_cu, as k_ffnn's is; by default at the two blocks that a CU holds.
 template <class T>
 static bool launch_ffnn_spread(const nepx_net* net, float scale, int d, const float* G, const int32_t* np_dev,
                                int64_t maxp, float* E, float* dEdG, void* stream) {
-    const int64_t tiles = (maxp + 15) / 16, cus = device_cus();
+    const int64_t tiles = (maxp + 15) / 16, cus = device_cus(), most = cus * tuning().net_blocks_per_cu;
     if (net->precision != NEPX_NET_F32 || (weights_in_lds<T, NEPX_NET_F32>() && tiles > 4 * cus)) return false;
     constexpr int TANH_NT = T::NL <= 2 ? 4 : 2, TANH_WV = TANH_NT == 4 && T::MT > 8 ? 8 : T::MT;
     constexpr int RELU_WV = T::MT > 8 ? 8 : T::MT;
 #define NEPX_LAUNCH_SPREAD(A, WV, NT)                                                                              \
-    hipLaunchKernelGGL((k_ffnn_spread<T, A, WV, NT>), dim3((unsigned)(tiles < 2 * cus ? tiles : 2 * cus)),         \
+    hipLaunchKernelGGL((k_ffnn_spread<T, A, WV, NT>), dim3((unsigned)(few ? tiles : most)),                        \
                        dim3((SpreadNet<T, A, WV, NT>::BLOCK)), 0, as_stream(stream), net->w_packed, net->en_min,   \
                        scale, d, G, np_dev, maxp, E, dEdG)
-    const bool few = tiles <= 2 * cus;  // one tile per block at most
+    const bool few = tiles <= most;  // one tile per block at most
     if (net->act == NEPX_ACT_TANH) {
         if (few) NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH, T::MT, 1);
         else NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH, TANH_WV, TANH_NT);

@@ -149,6 +149,38 @@ def test_ffnn_tile_groups_equal_single_tiles(gpu, d_in, widths, act):
         assert normwise_rel(dG[-500:].cpu().numpy(), 5.0 * want) < 1e-4
 
 
+@pytest.mark.parametrize("d_in,widths,act", [(121, [150] * 4, "relu"), (47, [150] * 4, "tanh"), (60, [128, 128], "tanh")])
+def test_ffnn_grid_follows_the_launch_tuning(gpu, d_in, widths, act):
+    """net_blocks_per_cu caps the grid of the network kernel that spreads layers over a block's waves, too; the
+    results are the same bits for any value."""
+    import ctypes as C
+    import nepx
+    from graph_util import kernel_launches
+    from nepx import _lib, tune
+    net = nepx.EnergyNet.random(d_in, widths, seed=5, act=act, device=gpu, precision="f32")
+    cn = net.cstruct()
+    P = 16 * 1300 - 3
+    G = 20.0 * torch.rand((P, d_in), generator=torch.Generator(device=gpu).manual_seed(4), device=gpu)
+    n_dev = torch.tensor([P], dtype=torch.int32, device=gpu)
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    old, res = tune.get_launch(), []
+    try:
+        for blocks in (1, 2, 4, 16):
+            tune.set_launch(tune.Tuning(**dict(old, net_blocks_per_cu=blocks)))
+            E, dG = torch.full((P,), float("nan"), device=gpu), torch.full((P, d_in), float("nan"), device=gpu)
+
+            def run(stream=None):
+                _lib.check(_lib.lib.nepx_ffnn_fwd_bwd(C.byref(cn), _lib.ptr(G), _lib.ptr(n_dev), P, _lib.ptr(E),
+                                                      _lib.ptr(dG), _lib.stream_handle(stream)), "nepx_ffnn_fwd_bwd")
+            assert kernel_launches(run)[0][0] == (min(1300, blocks * cus), 1, 1)
+            res.append((E, dG))
+    finally:
+        tune.set_launch(tune.Tuning(**old))
+    torch.cuda.synchronize()
+    for E, dG in res:
+        assert torch.isfinite(E).all() and torch.equal(E, res[0][0]) and torch.equal(dG, res[0][1])
+
+
 def test_ffnn_split_large_inputs_and_energy_range(gpu):
     """The fp16 hi/lo path with descriptor entries up to 4000 (|G| <= Nd^2 bounds real rows far
     below fp16's 65504) and an energy range of 5000: the backward deltas are carried without the
