@@ -1005,7 +1005,7 @@ static bool launch_ffnn_spread(const nepx_net* net, float scale, int d, const fl
                                int64_t maxp, float* E, float* dEdG, void* stream) {
     const int64_t tiles = (maxp + 15) / 16, cus = device_cus(), most = cus * tuning().net_blocks_per_cu;
     if (net->precision != NEPX_NET_F32 || (weights_in_lds<T, NEPX_NET_F32>() && tiles > 4 * cus)) return false;
-    constexpr int TANH_NT = T::NL <= 2 ? 4 : 2, TANH_WV = TANH_NT == 4 && T::MT > 8 ? 8 : T::MT;
+    constexpr int TANH_NT = T::NL <= 2 ? 4 : 2;
     constexpr int RELU_WV = T::MT > 8 ? 8 : T::MT;
 #define NEPX_LAUNCH_SPREAD(A, WV, NT)                                                                              \
     hipLaunchKernelGGL((k_ffnn_spread<T, A, WV, NT>), dim3((unsigned)(few ? tiles : most)),                        \
@@ -1014,7 +1014,7 @@ static bool launch_ffnn_spread(const nepx_net* net, float scale, int d, const fl
     const bool few = tiles <= most;  // one tile per block at most
     if (net->act == NEPX_ACT_TANH) {
         if (few) NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH, T::MT, 1);
-        else NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH, TANH_WV, TANH_NT);
+        else NEPX_LAUNCH_SPREAD(NEPX_ACT_TANH, T::MT, TANH_NT);
     } else {
         if (few) NEPX_LAUNCH_SPREAD(NEPX_ACT_RELU, T::MT, 1);
         else NEPX_LAUNCH_SPREAD(NEPX_ACT_RELU, RELU_WV, 4);

@@ -61,7 +61,8 @@ __device__ __forceinline__ void angular_site_grad_m(const HarmM<MS>& h, float ux
 }
 
 // The adjoint's sets: hypers 10 8 4 take two waves of 12 harmonics each, as one wave's sites would fill the
-// LDS of a whole SIMD's waves.
+// LDS of a whole SIMD's waves.  (One wave of all 24, each wave evaluating its own sites, took 50 (40) us at
+// 100,001 pairs of 12 (8) sites, but its sums lay further from 64 bits: 8.4e-7 against 8.0e-7 at 12 sites.)
 template <int LMAX>
 struct AdjSets : MGroups<LMAX> {};
 template <>
@@ -76,6 +77,7 @@ template <class Cfg>
 struct QuadAdj {
     using MG = AdjSets<Cfg::LMAX>;
     static constexpr int NA = Cfg::NANG + 1, NC = (NA + 3) / 4, STEPS = Cfg::ND / 4, BLOCK = 64 * MG::COUNT;
+    static_assert(MG::COUNT > 1, "the groups' sums meet in LDS");
     static constexpr bool OK = Cfg::ND % 4 == 0;
     // floats per pair of a trip's f and f' and of a wave's harmonics: strides of 4 odd keep the lanes' 64
     // scalar writes on 64 banks
@@ -296,22 +298,20 @@ __global__ __launch_bounds__((QuadAdj<Cfg>::BLOCK)) __attribute__((amdgpu_waves_
         float sum[12];
         static_for<COUNT>([&](auto gc) {
             constexpr int G = decltype(gc)::value;
-            if (COUNT == 1 || wave == G)
+            if (wave == G)
                 quad_adjoint_sums<Cfg, typename MG::template Set<G>, G == MG::RAD>(inv_rn, st, grow, xp, lane, sum);
         });
-        if (COUNT > 1 && q == 0) {
+        if (q == 0) {
 #pragma unroll
             for (int c = 0; c < 12; ++c) part[wave][c][slot] = sum[c];
         }
         __syncthreads();  // the groups' sums are there, and the rows and sites are used up
         if (wave == 0 && q == 0 && valid) {
-            if constexpr (COUNT > 1) {
 #pragma unroll
-                for (int c = 0; c < 12; ++c) {
-                    sum[c] = part[0][c][slot];
+            for (int c = 0; c < 12; ++c) {
+                sum[c] = part[0][c][slot];
 #pragma unroll
-                    for (int w = 1; w < COUNT; ++w) sum[c] += part[w][c][slot];
-                }
+                for (int w = 1; w < COUNT; ++w) sum[c] += part[w][c][slot];
             }
             AdjAcc acc;
             acc.G0x = sum[0]; acc.G0y = sum[1]; acc.G0z = sum[2];
