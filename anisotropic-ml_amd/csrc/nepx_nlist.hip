@@ -18,7 +18,7 @@ namespace nepx {
 
 constexpr int kNB = 256;        // threads per block
 constexpr int kScanBlock = 1024;
-constexpr int kSortMax = 2048;  // longest row the in-LDS sort accepts
+constexpr int kSortMax = 2048;  // longest row the sorts accept
 constexpr int kSlotsPerBlock = 1024;
 
 // One wrap of t: past L/2 either way, t moves L towards zero.  (The two tests t > L/2 -> t - L,
@@ -191,7 +191,8 @@ __global__ void k_cells_fill(nepx_state st, nepx_nlist nl) {
 //
 // LG: with 16 lanes a particle, 4,096 particles are one wave per SIMD and the walk waits for memory, so
 // systems of up to kWideGroups particles take a wave per particle (4,097 tetrahedra, a list of 402,000 pairs:
-// the two walks 254 -> 109 us, with cells of half the list radius as well).
+// the two walks 254 -> 84 us, with the columns walked as runs).  nepx/system.py picks the cells' side by the
+// lanes, so it holds this number as well.
 constexpr int kWideGroups = 8192;
 
 template <int LG>

@@ -11,8 +11,8 @@
 // trips dealt to the waves, and read from LDS.  The bound is VALU issue (site geometry, radial functions and the
 // per-site gradient sums) and, with two waves per SIMD, the waits of its chains.  8 (12) sites, hypers
 // 10 10 10: 241 pairs 45 -> 13 us (61 -> 13), 20,000 pairs 92 -> 46 us (128 -> 57), 100,001 pairs
-// 310 -> 189 us (419 -> 228); hypers 10 8 4: 241 pairs 15 -> 12 us (20 -> 13), 100,001 pairs 52 -> 47 us
-// (72 -> 59).
+// 300 -> 190 us (419 -> 230); hypers 10 8 4: 241 pairs 15 -> 13 us (20 -> 13), 100,001 pairs 52 -> 47 us
+// (71 -> 59); more than 896 pairs a CU of 8 sites go one to a lane (launch_adjoint).
 #pragma once
 #include "nepx_msets.h"
 #include "nepx_quad.h"

@@ -8,10 +8,10 @@
 //
 // One lane per cloud held at most 176 accumulators, so hypers 10 8 4 walked the sites twice and
 // 10 10 10 eight times, and its loads and stores strode by whole clouds and rows.  The bound is issue:
-// VALU work (radial functions, harmonics, sums of squares; 850 instructions per tile of 12 sites, hypers
+// VALU work (radial functions, harmonics, sums of squares; 865 instructions per tile of 12 sites, hypers
 // 10 8 4) and the products, next to the memory traffic.  12 sites: hypers 10 8 4, 1,000,003 clouds
-// 251 -> 153 us (2.2 TB/s), 5,000 clouds 18 -> 11 us; hypers 10 10 10, 1,373 -> 949 us, 5,000 clouds
-// 81 -> 12 us.
+// 252 -> 156 us (2.1 TB/s), 5,000 clouds 17 -> 11 us; hypers 10 10 10, 1,375 -> 977 us, 5,000 clouds
+// 80 -> 11 us.  Many clouds of a few sites stay one to a lane (launch_clouds).
 #pragma once
 #include "nepx_msets.h"
 #include "nepx_quad.h"
@@ -42,8 +42,8 @@ __device__ __forceinline__ void quad_cloud_sums(const float* pts, const float* _
                                                 float (&ga)[Cfg::NANG + 1][Cfg::LMAX], Done&& sites_done) {
     using Q = QuadCloud<Cfg>;
     constexpr int NC = Q::NC, NA = Q::NA, LC = (MS::N + 3) / 4, LMAX = Cfg::LMAX;
-    // The set's first l, a compile-time constant: found at run time it leaves the sums below in scratch memory, walked by
-    // loops (hypers 10 10 10: 50 us a tile, 50,000 clouds of 12 sites 325 us against 55 us).
+    // The set's first l, a compile-time constant: found at run time it leaves the sums below in scratch memory,
+    // walked by loops (hypers 10 10 10: 50 us a tile, 50,000 clouds of 12 sites 325 us against 55 us).
     constexpr int FIRST = MS::l_of(0);
     v4f Af[NC][LC];
 #pragma unroll

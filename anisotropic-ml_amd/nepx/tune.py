@@ -6,7 +6,7 @@ at FP32 rounding level):
   gather_lanes         lanes per particle in the deterministic force gather (4 .. 64)
   fused_blocks_per_cu  grid of the fused descriptor/network/adjoint kernel (persistent blocks per CU)
   pair_blocks_per_cu   grid cap of the split descriptor and adjoint kernels
-  net_blocks_per_cu    grid cap of the split network kernel
+  net_blocks_per_cu    grid cap of the split network kernels
   pair_lanes           lanes per pair in the fused kernel: 4 puts the per-pair site sums on the
                        matrix cores (default where the shape allows), 1 keeps one lane per pair;
                        the two differ in FP32 rounding only, so it is not searched by default

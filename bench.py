@@ -655,6 +655,10 @@ def main():
     peak = PEAK_FP32_MFMA_TFLOPS
     mfma_desc = NET_DESC[net.precision]
     prof = profiled(a.workload) if net.precision == "f16x3" else profiled(None)
+    # counters that show the VALU pipe idle more than half the time: the kernel waits (one wave per SIMD)
+    waits = prof["valu_issue_util"] is not None and prof["valu_issue_util"] < 0.5
+    if waits:
+        compute = compute.replace("the bound is FP32 VALU issue", "the bound is latency: one wave per SIMD waits")
     res = {
         "metric": ("particle-steps/s at 32k tetrahedra" if a.workload == "tet32k"
                    else f"particle-steps/s ({a.workload})"),
@@ -682,7 +686,7 @@ def main():
                                f"dt={w['dt']}",
                    "particles": spec.n, "pairs_per_step": P, "hipgraph": bool(a.graph),
                    "list_builds": int(flags[4]), "wall_s": wall},
-        "roofline": {"bound": "valu", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
+        "roofline": {"bound": "latency" if waits else "valu", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                      "frac": achieved / peak, "traffic": prof["traffic"],
                      "kernel": kernel, "kernel_ms": fused_ms, "compute": compute,
                      "flops_per_launch": flops, "flops_per_pair": pair_flops(shape.n_sites, hyp, D, widths),

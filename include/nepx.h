@@ -113,7 +113,8 @@ typedef struct nepx_nlist {
     int32_t* cell_list;              /* n               */
     double* cell_pos;                /* 4n: x, y, z of cell_list[k] at 4k..4k+2 (written by the build) */
     int32_t* cell_of;                /* n               */
-    int32_t* row_count;              /* n+1 (forward), then scanned to row_start  */
+    int32_t* row_count;              /* n+1: row lengths (explicit pair lists) or totals of the build's
+                                        blocks, scanned to row_start; rrow_count likewise */
     int32_t* row_start;              /* n+1 */
     int32_t* rrow_count;             /* n+1 */
     int32_t* rrow_start;             /* n+1 */
@@ -157,7 +158,7 @@ typedef struct nepx_tuning {
     int32_t fused_blocks_per_cu;   /* grid of the fused pair kernel = CUs x this (1..8; default 1)      */
     int32_t pair_blocks_per_cu;    /* grid cap of the descriptor / adjoint kernels (1..64; default 16)  */
     int32_t gather_lanes;          /* lanes per particle in the force gather: 4..64, power of 2 (16)   */
-    int32_t net_blocks_per_cu;     /* grid cap of the split network kernel (1..16; default 2)          */
+    int32_t net_blocks_per_cu;     /* grid cap of the split network kernels (1..16; default 2)         */
     int32_t pair_lanes;            /* lanes per pair in the fused kernel: 4 = site sums on MFMA where the
                                       shape allows (default), 1 = one lane per pair (site sums on VALU) */
 } nepx_tuning;
@@ -185,9 +186,9 @@ int nepx_net_pack_lowp(int32_t precision, int32_t d_in, int32_t width, int32_t n
 
 /* ---- descriptor, energy network, adjoint ------------------------------- */
 /* P = min(*n_pairs_dev, max_pairs) is read on the device; max_pairs sizes the launch.  Up to about
- * 2 x 64 pairs per CU (descriptor of multi-pass shapes) the work of one pair is spread over
- * several waves, and the FP32 network spreads its layers over a block's waves (up to 4 x 16 pairs per
- * CU, or any number for networks too wide for LDS); the results are the same bit for bit. */
+ * 2 x 64 pairs per CU (descriptor of multi-pass shapes, adjoint of the 12-site one) the work of one pair
+ * is spread over several waves, and the FP32 network spreads its layers over a block's waves (up to
+ * 4 x 16 pairs per CU, or any number for networks too wide for LDS); the results are the same bit for bit. */
 /* G (P x D, f32) of compacted pairs.  Replaces pos_to_pts + pts_to_nep_descriptors
  * (DescriptorGenerator.py:163-218,296-432); one row per pair (no FD stencil). */
 int nepx_descriptor_fwd(const nepx_pair_model* m, const float* qf, const int32_t* pair_i,
