@@ -59,8 +59,9 @@ def kind(op):
 
 
 def main_loop(body):
-    """Instructions of the main loop's body, in order: from the target of the last backward branch
-    to that branch."""
+    """Instructions of the main loop's body, in order: from the target of the innermost backward branches that
+    enclose every matrix product to the last of them.  (The loop's labels lie a few instructions apart; a branch
+    back from a block placed behind the loop, such as an early exit's, encloses the code before the loop as well.)"""
     labels, ins = {}, []
     for l in body[1:]:
         m = re.match(r"^(\.LBB\S+):", l)
@@ -74,8 +75,11 @@ def main_loop(body):
             if x.startswith(("s_branch", "s_cbranch")) and labels.get(x.split()[-1], len(ins)) < k]
     if not back:
         raise SystemExit("no main loop found")
-    end, head = max(back, key=lambda b: b[0] - b[1])
-    return ins[head:end + 1]
+    mfma = [k for k, x in enumerate(ins) if x.startswith("v_mfma")]
+    back = [b for b in back if not mfma or (b[1] <= mfma[0] and mfma[-1] <= b[0])] or back
+    inner = max(b[1] for b in back)
+    back = [b for b in back if b[1] > inner - 8]
+    return ins[min(b[1] for b in back):max(b[0] for b in back) + 1]
 
 
 def main():

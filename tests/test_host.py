@@ -633,3 +633,19 @@ def test_no_kernel_keeps_an_array_in_scratch_memory():
 def test_list_cells_take_the_shorter_walk(n, ratio, n_arena, nc):
     from nepx.system import _cells_per_side
     assert _cells_per_side(n, ratio * 3.0, 3.0, n_arena) == nc
+
+
+def test_isa_phases_cuts_the_innermost_loop_around_the_products():
+    """The main loop ends at its own last branch: neither at an earlier one (a skipped store) nor at a branch
+    back from a block that the compiler placed behind the loop."""
+    import importlib.util
+    path = os.path.join(ROOT, "anisotropic-ml_amd", "isa_phases.py")
+    spec = importlib.util.spec_from_file_location("isa_phases", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    body = (["_Zk:", "\ts_cbranch_scc0 .LBB0_4", ".LBB0_1:"] + ["\tv_mov_b32 v0, 0"] * 9 +
+            [".LBB0_2:", "\ts_nop 0", ".LBB0_3:", "\tv_add_f32 v1, v1, v1",
+             "\tv_mfma_f32_4x4x1_16b_f32 v[0:3], v4, v5, v[0:3]", "\ts_cbranch_execz .LBB0_3", "\tv_mul_f32 v1, v1, v1",
+             "\ts_branch .LBB0_2", ".LBB0_4:", "\ts_branch .LBB0_1"])
+    assert [x.split()[0] for x in mod.main_loop(body)] == ["s_nop", "v_add_f32", "v_mfma_f32_4x4x1_16b_f32",
+                                                           "s_cbranch_execz", "v_mul_f32", "s_branch"]
